@@ -31,10 +31,12 @@
 // src/ray/ray_core.h. Function comments cite the lines.
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
 #include "engine.h"
+#include "kd_pred.h"
 
 // Scan scratch of the allocation-free rasterization (btg_raster_device_noalloc):
 // row counts (4 B), span offsets (8 B) and tile sums for kNoAllocMaxPolys
@@ -67,7 +69,6 @@ constexpr int kMbox = 8;            // mailbox entries per lane (a power of two)
 enum App { kSoft = 0, kPrimary = 1, kPoint = 2, kSoftG = 3 };
 constexpr bool isSoft(int app) { return app == kSoft || app == kSoftG; }
 enum RootState { kTraced = 0, kKilled = 1, kNoBeam = 2 };
-enum { kNear = 0, kFar = 1, kBoth = 2 };
 enum { kKeep = 0, kAllIn = 1, kClip = 2 };
 enum { kFinished = 0, kSplit = 1, kContinue = 2 };
 enum { kDescend = 0, kTest = 1, kClimb = 2 };
@@ -210,6 +211,7 @@ struct Params {
   int tile, tilesW, cull;
   int leafCap;  // leaves a sub-beam may visit per trace launch before it yields (0: no cap)
   int mailbox;  // 1: per-lane mailbox of the triangles the lane's sub-beam has passed unchanged
+  int wideScene;  // 1: some scene's coordinates exceed kWide (or are NaN): kd predicates in the reference's arithmetic
   F3 pointLight;
   const OutPoly* prim;
   OutPoly* out;
@@ -372,13 +374,13 @@ __device__ __forceinline__ void setupQuery(RootQ& q, float extent) {
   q.farCq = dot(q.plane.n, q.plane.d);
 }
 
-// CoreBeam (beam_core.h:30-40).
+// CoreBeam (beam_core.h:30-40): the corners and direction signs. The rest of
+// the reference's fields (|w| per axis, the far plane) follow from them; see
+// Dirs and KdBounds.
 struct Beam {
-  C4 qx, qy, aw0, aw1, aw2, farA;
-  float farC;
+  C4 qx, qy;
   int n, hit;
   int s0, s1, s2;  // +-1 per axis
-  bool hasFar;
 };
 
 // Per-axis fields picked by value (a select of loaded values, never of
@@ -387,16 +389,6 @@ __device__ __forceinline__ int sgnOf(const Beam& b, int a) {
   const int s0 = b.s0, s1 = b.s1, s2 = b.s2;
   return a == 0 ? s0 : (a == 1 ? s1 : s2);
 }
-__device__ __forceinline__ C4 awOf(const Beam& b, int a) {
-  C4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = b.aw0.v[i], x1 = b.aw1.v[i], x2 = b.aw2.v[i];
-    r.v[i] = a == 0 ? x0 : (a == 1 ? x1 : x2);
-  }
-  return r;
-}
-
 // Plane of the current hit cached with the beam (WfWork, wavefront_core.h:58-61).
 struct Work {
   Beam b;
@@ -404,33 +396,6 @@ struct Work {
   F3 hitN;
 };
 
-// The beam's |w| per axis kept in the lane's LDS column as well (word
-// (4 a + i) * kBlock for axis a, corner i): the descent picks an axis per node
-// at run time, and reading that axis's four values from LDS costs no VALU
-// instruction, where selecting them among the registers of the three axes took
-// eight selects per axis.
-__device__ __forceinline__ C4 awAt(const float* awCol, int a) {
-  const float* q = awCol + a * 4 * kBlock;
-  return c4(q[0], q[kBlock], q[2 * kBlock], q[3 * kBlock]);
-}
-__device__ __forceinline__ void awStore(float* awCol, const Beam& b) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    awCol[i * kBlock] = b.aw0.v[i];
-    awCol[(4 + i) * kBlock] = b.aw1.v[i];
-    awCol[(8 + i) * kBlock] = b.aw2.v[i];
-  }
-}
-
-// Signed distances from the apex to a box's slabs along each axis, in the
-// rays' direction: nIn[k] to the face they enter by, nOut[k] to the face they
-// leave by (the Nmin / Nmax of beam_core.h:146-149, 171-173). The descent
-// carries them instead of the box: narrowing the box to a child moves one
-// face of the split axis onto the split plane, whose distance is the
-// descent's own Ns, so only that one value changes per kd step.
-struct SlabDist {
-  F3 nIn, nOut;
-};
 __device__ __forceinline__ SlabDist slabDist(const Ctx& c, const Beam& b, const Box& box) {
   SlabDist d;
 #pragma unroll
@@ -443,46 +408,10 @@ __device__ __forceinline__ SlabDist slabDist(const Ctx& c, const Beam& b, const 
   return d;
 }
 
-// decide (beam_core.h:139-164): near / far / both children of an inner node.
-__device__ int decide(const Beam& b, int a, float Ns, const SlabDist& sd, const float* awCol) {
-  const C4 awa = awAt(awCol, a);
-#pragma unroll
-  for (int k = 1; k <= 2; ++k) {
-    const int cc = a + k >= 3 ? a + k - 3 : a + k;
-    const C4 lhs = scaled(awAt(awCol, cc), Ns);
-    if (allBelow(lhs, scaled(awa, comp(sd.nIn, cc)), kKdRel)) return kFar;
-    if (allAbove(lhs, scaled(awa, comp(sd.nOut, cc)), kKdRel)) return kNear;
-  }
-  if (b.hasFar && allAbove(scaled(b.farA, Ns), scaled(awa, b.farC), kKdRel)) return kNear;
-  return kBoth;
-}
-
-// overlaps (beam_core.h:166-195): false if the beam certainly misses the box
-// whose slab distances are sd.
-__device__ bool overlaps(const Beam& b, const SlabDist& sd) {
-  const float nmin[3] = {sd.nIn.x, sd.nIn.y, sd.nIn.z}, nmax[3] = {sd.nOut.x, sd.nOut.y, sd.nOut.z};
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    if (nmax[k] < 0) return false;
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-#pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      if (k == e) continue;
-      if (allBelow(scaled(awOf(b, e), nmax[k]), scaled(awOf(b, k), nmin[e]), kKdRel)) return false;
-    }
-  if (b.hasFar) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (allAbove(scaled(b.farA, nmin[k]), scaled(awOf(b, k), b.farC), kKdRel)) return false;
-  }
-  return true;
-}
-__device__ __forceinline__ bool overlaps(const Ctx& c, const Beam& b, const Box& box) {
-  return overlaps(b, slabDist(c, b, box));
-}
-
-__device__ __forceinline__ void setAw(Beam& b, const Ctx& c) {
+// |w| per axis of the beam's corners (CoreBeam's aw, beam_core.h:200-221) and
+// its far plane (setStatus, beam_core.h:225-240): the current hit's plane, the
+// query's own for any-hit queries without a hit, or none.
+__device__ __forceinline__ void setAw(Dirs& d, const Beam& b, const Ctx& c) {
   const Plane& P = c.P;
   C4 w[3] = {affine(b.qx, P.u.x, b.qy, P.v.x, P.d.x), affine(b.qx, P.u.y, b.qy, P.v.y, P.d.y),
              affine(b.qx, P.u.z, b.qy, P.v.z, P.d.z)};
@@ -495,9 +424,27 @@ __device__ __forceinline__ void setAw(Beam& b, const Ctx& c) {
       const float ws = w[a].v[i] * float(sg[a]);
       aw[a].v[i] = 0.0f > ws ? 0.0f : ws;
     }
-  b.aw0 = aw[0];
-  b.aw1 = aw[1];
-  b.aw2 = aw[2];
+  d.aw0 = aw[0];
+  d.aw1 = aw[1];
+  d.aw2 = aw[2];
+}
+__device__ __forceinline__ void setFar(Dirs& d, const Ctx& c, const Beam& b, const float* A, float C) {
+  if (b.hit >= 0) {
+    const C4 f = affine(b.qx, A[0], b.qy, A[1], A[2]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d.farA.v[i] = __builtin_fabsf(f.v[i]);
+    d.farC = selAbs(C);
+    d.hasFar = true;
+  } else if (c.farIsPlane()) {
+    const float c0 = selAbs(c.farCq);
+    d.farA = splat(c0);
+    d.farC = c0;
+    d.hasFar = true;
+  } else {
+    d.farA = splat(0);
+    d.farC = 0;
+    d.hasFar = false;
+  }
 }
 
 // beamGeom (beam_core.h:200-221): corners (lanes past n repeat the last) and
@@ -521,28 +468,7 @@ __device__ __forceinline__ bool beamGeom(const Ctx& c, const Pg<N>& p, int s0, i
   b.s0 = s0;
   b.s1 = s1;
   b.s2 = s2;
-  setAw(b, c);
   return true;
-}
-
-// setStatus (beam_core.h:225-240).
-__device__ __forceinline__ void setStatus(const Ctx& c, Beam& b, int hit, const float* A, float C) {
-  b.hit = hit;
-  if (hit >= 0) {
-    const C4 f = affine(b.qx, A[0], b.qy, A[1], A[2]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b.farA.v[i] = __builtin_fabsf(f.v[i]);
-    b.farC = selAbs(C);
-    b.hasFar = true;
-  } else if (c.farIsPlane()) {
-    const float c0 = selAbs(c.farCq);
-    b.farA = splat(c0);
-    b.farC = c0;
-    b.hasFar = true;
-  } else {
-    b.farC = 0;
-    b.hasFar = false;
-  }
 }
 
 // hitPlane (beam_core.h:290-297) from the packed per-triangle normal/vertex.
@@ -554,6 +480,26 @@ __device__ __forceinline__ void hitPlane(const Params& p, const Ctx& c, int t, W
   w.hitA[1] = dot(nT, c.P.v);
   w.hitA[2] = dot(nT, c.P.d);
   w.hitC = dot(nT, relApex(c, f3(vv.x, vv.y, vv.z)));
+}
+
+__device__ __forceinline__ Dirs dirsOf(const Ctx& c, const Work& w) {
+  Dirs d;
+  setAw(d, w.b, c);
+  setFar(d, c, w.b, w.hitA, w.hitC);
+  return d;
+}
+
+// decide and overlaps by the beam's bounds; the reference's arithmetic, from
+// the corners, only where those leave it open.
+__device__ __forceinline__ int decideFast(const Ctx& c, const Work& w, int a, float Ns, const SlabDist& sd,
+                                          const float* col, bool slow) {
+  const int d = decideBounds<kBlock>(col, slow, a, Ns, sd);
+  return __builtin_expect(d == kBand, 0) ? decide(dirsOf(c, w), a, Ns, sd) : d;
+}
+__device__ __forceinline__ bool overlapsFast(const Ctx& c, const Work& w, const SlabDist& sd, const float* col,
+                                             bool slow) {
+  const int o = overlapsBounds<kBlock>(col, slow, sd);
+  return __builtin_expect(o == kBand, 0) ? overlaps(dirsOf(c, w), sd) : o != 0;
 }
 
 // wfExpand (wavefront_core.h:92-112). Any-hit applications (soft and point
@@ -572,15 +518,12 @@ __device__ void expand(const Params& p, const Ctx& c, const Rec& r, Work& w) {
   b.s0 = (r.negBits & 1) ? -1 : 1;
   b.s1 = (r.negBits & 2) ? -1 : 1;
   b.s2 = (r.negBits & 4) ? -1 : 1;
-  setAw(b, c);
-  const int hit = App == kPrimary ? r.hit : -1;
-  if (hit >= 0) {
-    hitPlane(p, c, hit, w);
-    setStatus(c, b, hit, w.hitA, w.hitC);
+  b.hit = App == kPrimary ? r.hit : -1;
+  if (b.hit >= 0) {
+    hitPlane(p, c, b.hit, w);
   } else {
     w.hitA[0] = w.hitA[1] = w.hitA[2] = w.hitC = 0;
     w.hitN = f3(0, 0, 0);
-    setStatus(c, b, -1, nullptr, 0);
   }
 }
 
@@ -1144,6 +1087,7 @@ struct Stepper {
   KdNodeD kn;                      // descend: node r.node
   uint32_t leafOffset, leafCount;  // the current leaf
   int validFrom;                   // path levels [validFrom, min(r.depth, kPathLevels)) are valid
+  bool slow;                       // the beam takes the reference's arithmetic for every kd predicate
 };
 
 // A lane's column of the LDS ancestor path: level k at col[k * kBlock] holds
@@ -1228,7 +1172,7 @@ struct PhaseClock {
 // Both children of an inner node are fetched while it is decided.
 template <int App>
 __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, const Path& path,
-                       const float* awCol, Cnt& cnt PHASE_ARG) {
+                       const float* bounds, Cnt& cnt PHASE_ARG) {
   const DevScene& sv = p.sv;
   const Beam& B = w.b;
   for (;;) {
@@ -1247,7 +1191,7 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
         const bool toRight = sga > 0;
         if (d < kPathLevels) path.set(d, toRight ? right : left);
         int dec = kFar;
-        if (Ns > 0) dec = decide(B, a, Ns, ss.sd, awCol);
+        if (Ns > 0) dec = decideFast(c, w, a, Ns, ss.sd, bounds, ss.slow);
         // kFar: into the child the rays move into; otherwise the apex side
         const bool goRight = (dec == kFar) == toRight;
         if (dec == kBoth) r.trail |= uint64_t(1) << d;
@@ -1312,7 +1256,7 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
       r.node = node;
       r.depth = int16_t(d);
       const SlabDist sd = slabDist(c, B, cb);
-      const bool ov = overlaps(B, sd);
+      const bool ov = overlapsFast(c, w, sd, bounds, ss.slow);
       PHASE_MARK(kPhBox);
       if (ov) {
         r.node = cs;
@@ -1327,11 +1271,22 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
   }
 }
 
+// A nearer hit (primary visibility) moves the beam's far plane.
+template <int App>
+__device__ __forceinline__ void farUpdate(const Ctx& c, const Work& w, Stepper& ss, float* bounds) {
+  KdBounds kb;
+  kb.slow = ss.slow;
+  farBounds<App != kPrimary>(dirsOf(c, w), kb);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) bounds[(3 * a + 2) * kBlock] = kb.far[a];
+  ss.slow = kb.slow;
+}
+
 // wfTestOne (wavefront_core.h:236-268). The excluded triangle (the shading
 // point's own) is skipped here, uncounted, as the reference skips it before
 // testing (wavefront_core.h:198, 276).
 template <int App>
-__device__ int testOne(const Params& p, const Ctx& c, Rec& r, Work& w, const Stepper& ss, Cnt& cnt) {
+__device__ int testOne(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, Cnt& cnt, float* bounds) {
   const uint32_t i = uint32_t(r.cursor);
   r.cursor = int32_t(i + 1);
   const LeafTri ref = p.sv.refs[ss.leafOffset + i];
@@ -1349,13 +1304,14 @@ __device__ int testOne(const Params& p, const Ctx& c, Rec& r, Work& w, const Ste
       emitOutput<App>(p, c, w.b, r.root, t, cnt);
       return kFinished;
     }
-    setStatus(c, w.b, t, ti.A, ti.C);
+    w.b.hit = t;
     w.hitA[0] = ti.A[0];
     w.hitA[1] = ti.A[1];
     w.hitA[2] = ti.A[2];
     w.hitC = ti.C;
     w.hitN = ti.n;
     r.hit = t;
+    farUpdate<App>(c, w, ss, bounds);
     return kContinue;
   }
   r.cursor = int32_t(i);
@@ -1406,8 +1362,8 @@ __device__ __forceinline__ C4 shflC4(const C4& v, int src) {
 // cleared whenever the lane's beam changes: a new record, or (primary) a
 // nearer hit. Results are the same with and without it.
 template <int App>
-__device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, const Stepper& ss, bool want,
-                        Cnt& cnt, int32_t* mboxLds) {
+__device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, bool want, Cnt& cnt,
+                        int32_t* mboxLds, float* bounds) {
   const int k = want ? int(ss.leafCount) - r.cursor : 0;
   int incl = k;
 #pragma unroll
@@ -1553,8 +1509,7 @@ __device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, const St
   if (first >= 0) {
     if (firstAllIn) {
       if (App == kPrimary) {  // testOne's nearest-hit update
-        const float A[3] = {hA0, hA1, hA2};
-        setStatus(c, w.b, firstTri, A, hC);
+        w.b.hit = firstTri;
         w.hitA[0] = hA0;
         w.hitA[1] = hA1;
         w.hitA[2] = hA2;
@@ -1562,6 +1517,7 @@ __device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, const St
         w.hitN = hN;
         r.hit = firstTri;
         r.cursor = first + 1;
+        farUpdate<App>(c, w, ss, bounds);
         if (p.mailbox) {  // a nearer hit: earlier Keeps were against the farther one
           int32_t* const own = mboxLds + threadIdx.x;
 #pragma unroll
@@ -1596,9 +1552,9 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
   Stepper ss;
   __shared__ uint32_t pathLds[kPathLevels * kBlock];
   __shared__ int32_t mboxLds[kMbox * kBlock];
-  __shared__ float awLds[12 * kBlock];
+  __shared__ float boundLds[kBoundWords * kBlock];
   const Path path{pathLds + threadIdx.x};
-  float* const awCol = awLds + threadIdx.x;
+  float* const bounds = boundLds + threadIdx.x;
   for (;;) {
     const uint64_t idle = __ballot(!active);
     const int nIdle = __popcll(idle);
@@ -1613,10 +1569,17 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
           } else {
             c = modeCtx<App>(p.roots[r.root]);
             expand<App>(p, c, r, w);
-            awStore(awCol, w.b);
+            const KdBounds kb = kdBounds<App != kPrimary>(dirsOf(c, w));
+            boundsStore<kBlock>(bounds, kb);
+            // coordinates that could overflow a product keep to the reference's arithmetic too
+            ss.slow = kb.slow || p.wideScene ||
+                      !(__builtin_fabsf(c.P.O.x) <= kWide && __builtin_fabsf(c.P.O.y) <= kWide &&
+                        __builtin_fabsf(c.P.O.z) <= kWide);
             if (r.cursor < 0) {
               ss.phase = kDescend;
               ss.sd = slabDist(c, w.b, p.sv.nodeBox[r.node]);
+              // an exit face behind the apex (never for a beam that overlaps its box) would turn a ratio's sign
+              ss.slow = ss.slow || ss.sd.nOut.x < 0 || ss.sd.nOut.y < 0 || ss.sd.nOut.z < 0;
               ss.kn = p.sv.nodes[r.node];
             } else {
               const KdNodeD kn = p.sv.nodes[r.node];
@@ -1641,15 +1604,15 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
     }
     PHASE_MARK(kPhRefill);
     int res = kContinue;
-    if (active) res = advance<App>(p, c, r, w, ss, path, awCol, cnt PHASE_PASS);
+    if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt PHASE_PASS);
     PHASE_MARK(kPhRest);
     if (kCoopTest) {
       const bool want = active && res == kContinue;  // a leaf with triangles pending
-      const int cr = coopTest<App>(p, c, r, w, ss, want, cnt, mboxLds);
+      const int cr = coopTest<App>(p, c, r, w, ss, want, cnt, mboxLds, bounds);
       if (want) res = cr;
     } else if (active) {
       while (res == kContinue) {
-        res = testOne<App>(p, c, r, w, ss, cnt);
+        res = testOne<App>(p, c, r, w, ss, cnt, bounds);
         if (res != kContinue || !moreInLeaf(ss, r)) break;
       }
     }
@@ -1982,9 +1945,12 @@ __device__ bool admitPiece(const Params& p, const Ctx& c, const Pg<8>& qd, const
     cnt.dropped += double(dropped);
     return true;
   }
-  setStatus(c, b, -1, nullptr, 0);
+  b.hit = -1;
   cnt.v[sRoots]++;
-  if (!overlaps(c, b, ao.bounds)) {
+  Dirs d;
+  setAw(d, b, c);
+  setFar(d, c, b, nullptr, 0);
+  if (!overlaps(d, slabDist(c, b, ao.bounds))) {
     emitOutput<App>(p, c, b, root, -1, cnt);
     return true;
   }
@@ -2893,6 +2859,12 @@ int prepare(Engine& e, int app, int R, int budget, Params& p, std::string& err) 
   // leaves (measured on the conference hall: 45 ms against 50 ms at 8).
   p.leafCap = app == kPrimary && e.opt.leafCap > 0 ? std::min(e.opt.leafCap, kPrimaryLeafCap) : e.opt.leafCap;
   p.mailbox = e.opt.mailbox;
+  for (const SceneRec& sr : e.scenes) {
+    if (!sr.live) continue;
+    const F3 v[2] = {sr.bounds.lo, sr.bounds.hi};
+    for (const F3& b : v)
+      if (!(std::fabs(b.x) <= kWide && std::fabs(b.y) <= kWide && std::fabs(b.z) <= kWide)) p.wideScene = 1;
+  }
   return 0;
 }
 
