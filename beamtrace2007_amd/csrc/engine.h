@@ -39,6 +39,13 @@ struct DevScene {
   const Box* nodeBox = nullptr;
   const uint32_t* parent = nullptr;
   const LeafTri* refs = nullptr;   // in leaf order (kd triIndices order)
+  // Per leaf its ancestors from the root down, (node, data word) each, from
+  // entry __float_as_uint(split) of the leaf's node: where a climb goes without
+  // following parent links, one load instead of a chain of about ten (8 B per
+  // leaf and level: 95 MB for the 2M-triangle building). Measured: sixteen blob
+  // and atrium jobs 925 -> 878 ms, the plant at 512 x 512 117 -> 112 ms, primary
+  // and point shadows of the building 21.3 -> 19.7 ms. Null: no lists.
+  const uint2* anc = nullptr;
   const int32_t* refTri = nullptr; // the triangle id of each leaf reference (the mailbox's 4-byte read)
   Box bounds;                      // kd root box
   int numTris = 0;

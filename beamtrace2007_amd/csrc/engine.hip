@@ -1086,6 +1086,7 @@ struct Stepper {
   SlabDist sd;                     // descend: slab distances of r.node's box
   KdNodeD kn;                      // descend: node r.node
   uint32_t leafOffset, leafCount;  // the current leaf
+  uint32_t ancBase;                // its ancestors' entries in DevScene::anc (the last leaf's, during a climb)
   int validFrom;                   // path levels [validFrom, min(r.depth, kPathLevels)) are valid
   bool slow;                       // the beam takes the reference's arithmetic for every kd predicate
 };
@@ -1166,8 +1167,10 @@ struct PhaseClock {
 // triangle, climb to the next pending far child; returns kContinue with a
 // triangle pending at r.cursor, or kFinished after emitting the output.
 // The descent records each ancestor's far child in the lane's LDS path, so a
-// climb reads the pending child there and fetches its box, its parent and
-// the child itself at once, instead of following parent links; the climb
+// climb reads the pending child there and fetches its box and the child
+// itself at once; a level the path does not hold (a record resumed from a
+// queue starts with an empty one) is read from the leaf's ancestor list, one
+// load instead of a chain of parent links as long as the climb. The climb
 // counter still adds one per level climbed, as the reference's walk does.
 // Both children of an inner node are fetched while it is decided.
 template <int App>
@@ -1208,6 +1211,7 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
       cnt.v[sLeaf]++;
       ss.leafOffset = kn.offset;
       ss.leafCount = kn.data >> 2;
+      ss.ancBase = __float_as_uint(kn.split);
       ss.phase = kTest;
       PHASE_MARK(kPhDescend);
     }
@@ -1229,31 +1233,21 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
       if (d >= ss.validFrom && d < kPathLevels) {
         cs = path.get(d);
       } else {
-        // parent links from the shallowest known ancestor below depth d (the
-        // parent of a recorded far child, or r.node) up to depth d
-        int depth = r.depth;
-        uint32_t node = r.node;
-        if (d < ss.validFrom && ss.validFrom < depth && ss.validFrom < kPathLevels) {
-          depth = ss.validFrom;
-          node = sv.parent[path.get(depth)];
+        uint2 e;  // the ancestor at depth d: its node number and data word
+        if (sv.anc) {
+          e = sv.anc[size_t(ss.ancBase) + uint32_t(d)];
+        } else {  // no lists (see DevScene::anc): parent links up from the current node
+          uint32_t node = r.node;
+          for (int k = r.depth; k > d; --k) node = sv.parent[node];
+          e = make_uint2(node, sv.nodes[node].data);
         }
-        while (depth > d) {
-          node = sv.parent[node];
-          --depth;
-        }
-        const KdNodeD kn = sv.nodes[node];
-        cs = sgnOf(B, int(kn.data & 3u)) > 0 ? (kn.data >> 2) : node + 1;
-        if (d < kPathLevels) {
-          path.set(d, cs);
-          ss.validFrom = d;
-        }
+        cs = sgnOf(B, int(e.y & 3u)) > 0 ? (e.y >> 2) : e.x + 1;
+        if (d < ss.validFrom) ss.validFrom = d + 1;
       }
       PHASE_MARK(kPhWalk);
       r.trail &= (uint64_t(1) << d) - 1;
       const Box cb = sv.nodeBox[cs];
-      const uint32_t node = sv.parent[cs];
       const KdNodeD kc = sv.nodes[cs];
-      r.node = node;
       r.depth = int16_t(d);
       const SlabDist sd = slabDist(c, B, cb);
       const bool ov = overlapsFast(c, w, sd, bounds, ss.slow);
@@ -1267,6 +1261,7 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
         ss.kn = kc;
         break;
       }
+      if (!sv.anc) r.node = sv.parent[cs];
     }
   }
 }
@@ -1585,6 +1580,7 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
               const KdNodeD kn = p.sv.nodes[r.node];
               ss.leafOffset = kn.offset;
               ss.leafCount = kn.data >> 2;
+              ss.ancBase = __float_as_uint(kn.split);
               ss.phase = kTest;
             }
             ss.validFrom = r.depth;
@@ -2724,6 +2720,7 @@ struct SceneRec {
   int numTris = 0;
   uint32_t numVerts = 0;
   float offset = 0, offsetGuard = 0;
+  uint64_t ancEntries = 0;  // ancestor list entries of its leaves
   uint32_t nodeBase = 0, refBase = 0, triBase = 0, vertBase = 0;  // placement in the arena
 };
 
@@ -2736,7 +2733,7 @@ class Engine {
   hipEvent_t ev[4] = {};
   int cus = 0;
   // scene storage
-  void* sceneMem[6] = {};
+  void* sceneMem[7] = {};
   // engine buffers (grown on demand)
   DevBuf tq0, tq1, sq, roots, live, state, epoch, missFx, gFx, stats, st, out, outRoot, outTag, list, listCount;
   DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, prim, retry, cycles, shq, jobs;
@@ -3110,6 +3107,19 @@ SceneRec makeSceneRec(const btg_scene_desc& d, float offset, float offsetGuard) 
   return sr;
 }
 
+// Each leaf's ancestors, root first, at the base its split field holds: the
+// leaf's depth entries of (node, data word).
+__global__ void fillAncestors(DevScene sv, uint32_t nodes, uint2* anc) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nodes) return;
+  const KdNodeD leaf = sv.nodes[i];
+  if ((leaf.data & 3u) != 3u) return;
+  uint32_t depth = 0;
+  for (uint32_t k = i, up; (up = sv.parent[k]) != k; k = up) ++depth;
+  uint2* const list = anc + __float_as_uint(leaf.split);
+  for (uint32_t k = sv.parent[i], d = depth; d-- > 0; k = sv.parent[k]) list[d] = make_uint2(k, sv.nodes[k].data);
+}
+
 // Concatenates the live scenes into the device arena. Node, leaf-reference,
 // triangle and vertex numbers of each scene are shifted by its base; the
 // order of a triangle's vertex numbers (which orients shared edges) is kept.
@@ -3138,24 +3148,35 @@ int rebuildArena(Engine& e, std::string& err) {
   std::vector<uint32_t> par;
   std::vector<LeafTri> lt;
   std::vector<int32_t> rt;
+  std::vector<uint32_t> depths;  // of the arena's nodes (a parent is numbered before its children)
+  uint64_t ancEntries = 0;
+  depths.reserve(nodes);
   nv.reserve(size_t(tris) * 2);
   kn.reserve(nodes);
   bx.reserve(nodes);
   par.reserve(nodes);
   lt.reserve(refs);
   rt.reserve(refs);
-  for (const SceneRec& sr : e.scenes) {
+  for (SceneRec& sr : e.scenes) {
     if (!sr.live) continue;
+    const uint64_t anc0 = ancEntries;
     nv.insert(nv.end(), sr.triNV.begin(), sr.triNV.end());
     for (size_t i = 0; i < sr.nodes.size(); ++i) {
       KdNodeD n = sr.nodes[i];
-      if ((n.data & 3u) != 3u)
+      const uint32_t depth = i == 0 ? 0u : depths[sr.nodeBase + sr.parent[i]] + 1u;
+      depths.push_back(depth);
+      if ((n.data & 3u) != 3u) {
         n.data = (n.data & 3u) | (((n.data >> 2) + sr.nodeBase) << 2);
-      else
+      } else {
         n.offset += sr.refBase;
+        const uint32_t base = uint32_t(ancEntries);  // a leaf's split field is unused: its ancestors' first entry
+        std::memcpy(&n.split, &base, sizeof(base));
+        ancEntries += depth;
+      }
       kn.push_back(n);
       par.push_back(i == 0 ? sr.nodeBase : sr.parent[i] + sr.nodeBase);
     }
+    sr.ancEntries = ancEntries - anc0;
     bx.insert(bx.end(), sr.boxes.begin(), sr.boxes.end());
     for (LeafTri r : sr.refs) {
       r.tri += int32_t(sr.triBase);
@@ -3177,6 +3198,22 @@ int rebuildArena(Engine& e, std::string& err) {
   if (!rc) rc = upload(e, 4, lt.data(), lt.size(), sv.refs, err);
   if (!rc) rc = upload(e, 5, rt.data(), rt.size(), sv.refTri, err);
   if (rc) return rc;
+  // The ancestor lists are filled on the device from the parent links. Without
+  // room for them (or with more entries than 32 bits number) climbs follow
+  // the parent links instead.
+  sv.anc = nullptr;
+  if (ancEntries > 0 && ancEntries < (1ull << 32)) {
+    void* d = nullptr;
+    if (hipMalloc(&d, size_t(ancEntries) * sizeof(uint2)) == hipSuccess) {
+      e.sceneMem[6] = d;
+      fillAncestors<<<(nodes + 255) / 256, 256, 0, e.stream>>>(sv, nodes, static_cast<uint2*>(d));
+      BTG_TRY(hipGetLastError());
+      BTG_TRY(hipStreamSynchronize(e.stream));
+      sv.anc = static_cast<const uint2*>(d);
+    } else {
+      (void)hipGetLastError();
+    }
+  }
   const SceneRec& s0 = e.scenes[0];
   sv.bounds = s0.bounds;
   sv.numTris = s0.numTris;
@@ -3292,7 +3329,7 @@ int64_t engineSceneBytes(const Engine* e, int scene) {
   if (scene < 0 || size_t(scene) >= e->scenes.size() || !e->scenes[size_t(scene)].live) return -1;
   const SceneRec& sr = e->scenes[size_t(scene)];
   return int64_t(sr.triNV.size() * sizeof(float4) + sr.nodes.size() * (sizeof(KdNodeD) + sizeof(Box) + 4) +
-                 sr.refs.size() * (sizeof(LeafTri) + sizeof(int32_t)));
+                 sr.refs.size() * (sizeof(LeafTri) + sizeof(int32_t)) + sr.ancEntries * sizeof(uint2));
 }
 
 // roots: RootQ, live, state, epoch, missFx, gFx (as prepare allocates them)
