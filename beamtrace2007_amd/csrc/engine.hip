@@ -14,7 +14,9 @@
 //                 pieces (so the wave reserves exactly the queue slots it
 //                 needs with one atomic), then writing them in place - no
 //                 per-lane piece buffer.
-// The last workgroup of splitKernel to finish schedules the next round
+// A round whose queue does not fill the device runs as one launch after the
+// admission instead (waveKernel).
+// The last workgroup of a round's last launch to finish schedules the next round
 // (admission by reserved budget, as the reference's scheduleKernel,
 // cuda/wavefront.cu:327-345), so no single-thread launch is needed.
 //
@@ -125,7 +127,6 @@ struct WState {
   int admitBegin, admitCount;
   int done;
   int maxQueue;
-  int overflow;
   int round;
   unsigned long long traceItems, splitItems;
   LineInts<2> count;  // records in the trace queues (ping-pong by round)
@@ -178,9 +179,11 @@ struct Params {
   int R;
   const int* rootList;
   int budget;
+  int reserve;  // queue records set aside per admitted root until it is done
   unsigned long long capacity;
   Rec* tq[2];
   Rec* sq;
+  char* ws;  // fused passes: kWsBytes of buffers per wave of the grid (null: rounds of separate launches)
   RootQ* roots;
   int* live;
   int* state;
@@ -604,7 +607,7 @@ __device__ __forceinline__ TriS triSetup(const Ctx& c, const LeafTri& ref) {
 }
 
 // closerLine (beam_core.h:302-317).
-__device__ Ln closerLine(const Ctx& c, const TriS& T, const float* AF, float CF, F3 nF, int fId) {
+__device__ __forceinline__ Ln closerLine(const Ctx& c, const TriS& T, const float* AF, float CF, F3 nF, int fId) {
   const float cosang = dot(T.n, nF);
   const float scaleC = selMax(selAbs(T.C), selAbs(CF));
   const float ca = selAbs(cosang);
@@ -617,7 +620,7 @@ __device__ Ln closerLine(const Ctx& c, const TriS& T, const float* AF, float CF,
 
 // separated (beam_core.h:321-342): some beam side plane has all three
 // vertices strictly outside. Lane k holds side k -> k+1 (the reference's rot1).
-__device__ bool separated(const Ctx& c, const Beam& b, const TriS& ti) {
+__device__ __forceinline__ bool separated(const Ctx& c, const Beam& b, const TriS& ti) {
   const Plane& P = c.P;
   const C4 wx = affine(b.qx, P.u.x, b.qy, P.v.x, P.d.x);
   const C4 wy = affine(b.qx, P.u.y, b.qy, P.v.y, P.d.y);
@@ -703,7 +706,7 @@ __device__ __forceinline__ int classifyTri(const Ctx& c, const Work& w, const Tr
 
 // classifyTri for the trace kernel with the lazy setup: the same decisions as
 // classifyTri (beam_core.h:374-409), computing each line only when reached.
-__device__ int classifyLazy(const Ctx& c, const Work& w, TriS& ti) {
+__device__ __forceinline__ int classifyLazy(const Ctx& c, const Work& w, TriS& ti) {
   const Beam& B = w.b;
   bool allIn = true;
   int r = lineTest(c, B, triEdge<0>(c, ti));
@@ -931,7 +934,7 @@ __device__ __forceinline__ double pow2(int e) { return __builtin_ldexp(1.0, e); 
 
 // polygonFormFactorG (soft_core.h:18-33) of a 3- or 4-gon, unrolled with
 // constant indices so that the corners stay in registers.
-__device__ float formFactor(F3 x, F3 n, const F3 (&poly)[4], int count) {
+__device__ __forceinline__ float formFactor(F3 x, F3 n, const F3 (&poly)[4], int count) {
   double sum = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -964,7 +967,7 @@ __device__ __forceinline__ float area4(const C4& x, const C4& y) {
 
 // Appends an output polygon (primary / point shadows); the active lanes of a
 // wave share one atomic.
-__device__ void appendPoly(const Params& p, int root, const OutPoly& ob) {
+__device__ __forceinline__ void appendPoly(const Params& p, int root, const OutPoly& ob) {
   const int k = activeAppend(&p.st->outCount);
   if (k >= p.outCap) return;  // the host traces again with a larger buffer
   p.out[k] = ob;
@@ -975,7 +978,7 @@ __device__ void appendPoly(const Params& p, int root, const OutPoly& ob) {
 // pointShadowToImage (point_core.h:41-64) of a 3- or 4-gon on the receiver
 // plane sp: project to the image plane, make it counter-clockwise, repeat the
 // last corner.
-__device__ bool pointToImage(const Plane& camPlane, const Plane& sp, const C4& sx, const C4& sy, int n, int T,
+__device__ __forceinline__ bool pointToImage(const Plane& camPlane, const Plane& sp, const C4& sx, const C4& sy, int n, int T,
                              OutPoly& ip) {
   ip.n = n;
   ip.tri = T;
@@ -1006,10 +1009,34 @@ __device__ bool pointToImage(const Plane& camPlane, const Plane& sp, const C4& s
   return true;
 }
 
+// ---------------------------------------------------------- root budgets
+__device__ int jobOfRoot(const Params& p, int k);
+
+// A root has no live sub-beam left: release its budget reservation and, in an
+// open pass, count it off its job.
+__device__ __forceinline__ void rootDone(const Params& p, int root) {
+  atomicAdd(&p.st->reserved, (unsigned long long)(-(long long)p.reserve));
+  if (p.jobLeft) atomicSub(&p.jobLeft[jobOfRoot(p, root)], 1);
+}
+__device__ __forceinline__ void liveSub(const Params& p, int root, int n) {
+  if (atomicSub(&p.live[root], n) == n) rootDone(p, root);
+}
+__device__ __forceinline__ void killRoot(const Params& p, int root) {
+  if (atomicExch(&p.state[root], int(kKilled)) != int(kKilled)) atomicAdd(&p.st->killed, 1);
+}
+
+// Where a wave of the fused kernel puts the pieces that wait for their Lambert
+// integral: its own buffer and the LDS count of them (null: the pass's queue).
+struct WaveShade {
+  ShadeRec* buf;
+  int* count;
+};
+
 // A finished piece (wfOutput, wavefront_core.h:124-132, and the per-app
 // handling of cuda/wavefront.cu:193-227).
 template <int App>
-__device__ __forceinline__ void emitOutput(const Params& p, const Ctx& c, const Beam& b, int root, int tri, Cnt& cnt) {
+__device__ __forceinline__ void emitOutput(const Params& p, const Ctx& c, const Beam& b, int root, int tri, Cnt& cnt,
+                                           WaveShade wsh = WaveShade{nullptr, nullptr}) {
   const float area = area4(b.qx, b.qy);
   if (tri >= 0) cnt.v[sHits]++;
   cnt.v[sBeams]++;
@@ -1017,20 +1044,23 @@ __device__ __forceinline__ void emitOutput(const Params& p, const Ctx& c, const 
     if (tri >= 0) return;  // occluded
     const RootQ& R = p.roots[root];
     if (area > 0) atomicAdd(&p.missFx[root], (unsigned long long)(double(area) * pow2(-R.unitExp)));
-    if (p.exact) {  // the Lambert integral is taken by shadeKernel, after this round's trace
-      const int k = activeAppend(&p.st->shadeCount);
-      if ((unsigned long long)k < p.capacity) {
-        ShadeRec sr;
+    if (p.exact) {  // the Lambert integral is taken later, by full waves (shadeOne)
+      ShadeRec sr;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sr.qx[i] = b.qx.v[i];
-          sr.qy[i] = b.qy.v[i];
-        }
-        sr.root = root;
-        sr.n = b.n;
-        p.shq[k] = sr;
+      for (int i = 0; i < 4; ++i) {
+        sr.qx[i] = b.qx.v[i];
+        sr.qy[i] = b.qy.v[i];
+      }
+      sr.root = root;
+      sr.n = b.n;
+      if (wsh.buf) {  // room for a piece per lane is made before every step
+        wsh.buf[atomicAdd(wsh.count, 1)] = sr;
       } else {
-        p.st->overflow = 1;
+        const int k = activeAppend(&p.st->shadeCount);
+        if ((unsigned long long)k < p.capacity)
+          p.shq[k] = sr;
+        else
+          killRoot(p, root);
       }
     }
     return;
@@ -1054,20 +1084,32 @@ __device__ __forceinline__ void emitOutput(const Params& p, const Ctx& c, const 
   appendPoly(p, root, ob);
 }
 
-// ---------------------------------------------------------- root budgets
-__device__ int jobOfRoot(const Params& p, int k);
-
-// A root has no live sub-beam left: release its budget reservation and, in an
-// open pass, count it off its job.
-__device__ __forceinline__ void rootDone(const Params& p, int root) {
-  atomicAdd(&p.st->reserved, (unsigned long long)(-(long long)p.budget));
-  if (p.jobLeft) atomicSub(&p.jobLeft[jobOfRoot(p, root)], 1);
+// Records and pieces that find no room in a queue: their root is abandoned, to
+// be traced again. A pass's first run sets aside fewer records per root than
+// its budget (Params::reserve), so this can happen there; a retry reserves the
+// whole budget.
+__device__ __forceinline__ void toQueue(const Params& p, int q, int slot, const Rec& r) {
+  if ((unsigned long long)slot < p.capacity) {
+    p.tq[q][slot] = r;
+  } else {
+    killRoot(p, r.root);
+    liveSub(p, r.root, 1);
+  }
 }
-__device__ __forceinline__ void liveSub(const Params& p, int root, int n) {
-  if (atomicSub(&p.live[root], n) == n) rootDone(p, root);
-}
-__device__ __forceinline__ void killRoot(const Params& p, int root) {
-  if (atomicExch(&p.state[root], int(kKilled)) != int(kKilled)) atomicAdd(&p.st->killed, 1);
+// `slots` records from `slot` on; null if they do not all fit (the ones that do
+// then hold dropped slivers of the root).
+__device__ __forceinline__ Rec* roomAt(const Params& p, int q, int slot, int slots, int root) {
+  if ((unsigned long long)(slot + slots) <= p.capacity) return p.tq[q] + slot;
+  if (slots > 0) {
+    killRoot(p, root);
+    int lost = slots;
+    for (int k = 0; k < slots && (unsigned long long)(slot + k) < p.capacity; ++k, --lost) {
+      p.tq[q][slot + k].n = 0;
+      p.tq[q][slot + k].root = root;
+    }
+    if (lost > 0) liveSub(p, root, lost);
+  }
+  return nullptr;
 }
 
 // ------------------------------------------------------------- the trace
@@ -1174,8 +1216,8 @@ struct PhaseClock {
 // counter still adds one per level climbed, as the reference's walk does.
 // Both children of an inner node are fetched while it is decided.
 template <int App>
-__device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, const Path& path,
-                       const float* bounds, Cnt& cnt PHASE_ARG) {
+__device__ __forceinline__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, const Path& path,
+                       const float* bounds, Cnt& cnt, WaveShade wsh PHASE_ARG) {
   const DevScene& sv = p.sv;
   const Beam& B = w.b;
   for (;;) {
@@ -1222,7 +1264,7 @@ __device__ int advance(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& 
     for (;;) {
       if (r.trail == 0) {
         PHASE_MARK(kPhRest);
-        emitOutput<App>(p, c, B, r.root, c.anyHit() ? -1 : B.hit, cnt);
+        emitOutput<App>(p, c, B, r.root, c.anyHit() ? -1 : B.hit, cnt, wsh);
         PHASE_MARK(kPhEmit);
         return kFinished;
       }
@@ -1357,7 +1399,7 @@ __device__ __forceinline__ C4 shflC4(const C4& v, int src) {
 // cleared whenever the lane's beam changes: a new record, or (primary) a
 // nearer hit. Results are the same with and without it.
 template <int App>
-__device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, bool want, Cnt& cnt,
+__device__ __forceinline__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper& ss, bool want, Cnt& cnt,
                         int32_t* mboxLds, float* bounds) {
   const int k = want ? int(ss.leafCount) - r.cursor : 0;
   int incl = k;
@@ -1403,7 +1445,8 @@ __device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper&
     oc.eps = __shfl(c.eps, owner, kWave);
     oc.minArea = 0;
     oc.farCq = __shfl(c.farCq, owner, kWave);
-    oc.flags = App == kPrimary ? __shfl(c.flags, owner, kWave) : c.flags;
+    // (a lane that never held a beam has no flags of its own)
+    oc.flags = App == kPrimary ? __shfl(c.flags, owner, kWave) : (fAnyHit | fFarIsPlane);
     oc.exclude = __shfl(c.exclude, owner, kWave);
     Work ow;
     ow.b.qx = shflC4(w.b.qx, owner);
@@ -1530,6 +1573,44 @@ __device__ int coopTest(const Params& p, const Ctx& c, Rec& r, Work& w, Stepper&
   return kContinue;
 }
 
+// Makes record r the lane's sub-beam (false: a dropped sliver or an abandoned
+// root's, which only leaves its root's live count).
+template <int App>
+__device__ __forceinline__ bool loadBeam(const Params& p, Ctx& c, const Rec& r, Work& w, Stepper& ss, float* bounds,
+                                         int32_t* mboxLds) {
+  if (r.n == 0 || p.state[r.root] == kKilled) {
+    liveSub(p, r.root, 1);
+    return false;
+  }
+  c = modeCtx<App>(p.roots[r.root]);
+  expand<App>(p, c, r, w);
+  const KdBounds kb = kdBounds<App != kPrimary>(dirsOf(c, w));
+  boundsStore<kBlock>(bounds, kb);
+  // coordinates that could overflow a product keep to the reference's arithmetic too
+  ss.slow = kb.slow || p.wideScene ||
+            !(__builtin_fabsf(c.P.O.x) <= kWide && __builtin_fabsf(c.P.O.y) <= kWide &&
+              __builtin_fabsf(c.P.O.z) <= kWide);
+  const KdNodeD kn = p.sv.nodes[r.node];
+  if (r.cursor < 0) {
+    ss.phase = kDescend;
+    ss.sd = slabDist(c, w.b, p.sv.nodeBox[r.node]);
+    // an exit face behind the apex (never for a beam that overlaps its box) would turn a ratio's sign
+    ss.slow = ss.slow || ss.sd.nOut.x < 0 || ss.sd.nOut.y < 0 || ss.sd.nOut.z < 0;
+    ss.kn = kn;
+  } else {
+    ss.leafOffset = kn.offset;
+    ss.leafCount = kn.data >> 2;
+    ss.ancBase = __float_as_uint(kn.split);
+    ss.phase = kTest;
+  }
+  ss.validFrom = r.depth;
+  if (p.mailbox) {
+#pragma unroll
+    for (int k = 0; k < kMbox; ++k) mboxLds[k * kBlock + threadIdx.x] = -1;
+  }
+  return true;
+}
+
 template <int App>
 __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, int cur) {
   Cnt cnt;
@@ -1559,38 +1640,8 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
         const int i = base + rankBelow(idle);
         if (i < n) {
           r = q[i];
-          if (r.n == 0 || p.state[r.root] == kKilled) {  // a dropped sliver, or an abandoned root
-            liveSub(p, r.root, 1);
-          } else {
-            c = modeCtx<App>(p.roots[r.root]);
-            expand<App>(p, c, r, w);
-            const KdBounds kb = kdBounds<App != kPrimary>(dirsOf(c, w));
-            boundsStore<kBlock>(bounds, kb);
-            // coordinates that could overflow a product keep to the reference's arithmetic too
-            ss.slow = kb.slow || p.wideScene ||
-                      !(__builtin_fabsf(c.P.O.x) <= kWide && __builtin_fabsf(c.P.O.y) <= kWide &&
-                        __builtin_fabsf(c.P.O.z) <= kWide);
-            if (r.cursor < 0) {
-              ss.phase = kDescend;
-              ss.sd = slabDist(c, w.b, p.sv.nodeBox[r.node]);
-              // an exit face behind the apex (never for a beam that overlaps its box) would turn a ratio's sign
-              ss.slow = ss.slow || ss.sd.nOut.x < 0 || ss.sd.nOut.y < 0 || ss.sd.nOut.z < 0;
-              ss.kn = p.sv.nodes[r.node];
-            } else {
-              const KdNodeD kn = p.sv.nodes[r.node];
-              ss.leafOffset = kn.offset;
-              ss.leafCount = kn.data >> 2;
-              ss.ancBase = __float_as_uint(kn.split);
-              ss.phase = kTest;
-            }
-            ss.validFrom = r.depth;
-            active = true;
-            leaves = 0;
-            if (p.mailbox) {
-#pragma unroll
-              for (int k = 0; k < kMbox; ++k) mboxLds[k * kBlock + threadIdx.x] = -1;
-            }
-          }
+          active = loadBeam<App>(p, c, r, w, ss, bounds, mboxLds);
+          leaves = 0;
         }
       }
     }
@@ -1600,7 +1651,7 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
     }
     PHASE_MARK(kPhRefill);
     int res = kContinue;
-    if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt PHASE_PASS);
+    if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt, WaveShade{nullptr, nullptr} PHASE_PASS);
     PHASE_MARK(kPhRest);
     if (kCoopTest) {
       const bool want = active && res == kContinue;  // a leaf with triangles pending
@@ -1627,11 +1678,7 @@ __global__ void __launch_bounds__(kBlock) TRACE_OCCUPANCY traceKernel(Params p, 
       base = __shfl(base, 0, kWave);
       if (yield) {
         storeGeom(w.b, r);
-        const int slot = base + rankBelow(yields);
-        if ((unsigned long long)slot < p.capacity)
-          p.tq[cur ^ 1][slot] = r;
-        else
-          p.st->overflow = 1;
+        toQueue(p, cur ^ 1, base + rankBelow(yields), r);
         active = false;
       }
     }
@@ -1712,113 +1759,108 @@ struct EmitSink {
 
 __device__ void scheduleNext(const Params& p, int cur);
 
-template <int App>
-__global__ void __launch_bounds__(kBlock) SPLIT_OCCUPANCY splitKernel(Params p, int cur) {
-  Cnt cnt;
-  cnt.zero();
-  __shared__ float stageLds[kStageSlots * kStageWords * kBlock];
-  float* const stageCol = stageLds + threadIdx.x;
-  const int n = int(min((unsigned long long)p.st->splitCount, p.capacity));
-  const int nxt = cur ^ 1;
-  const Deal dl = dealOf();
-  bool first = true, exhausted = false;
-  while (n > 0 && !exhausted) {  // an empty round skips to the scheduling below
-    const int base = nextChunk(dl, &p.st->head[kHeadSplit], kWave, n, first, exhausted);
-    if (base >= n) break;
-    const int i = base + lane();
-    int slots = 0;
-    bool have = false, emit = false, commit = false;
-    Rec r;
-    Work w;
-    Ctx c;
-    Ln L[5];
-    int nl = 0;
-    int recs0 = 0;
-    int staged = -1;  // pieces kept in LDS by the counting pass (-1: clip again)
-    int tri = -1;
-    if (i < n) {
-      r = p.sq[i];
-      if (p.state[r.root] == kKilled) {
-        liveSub(p, r.root, 1);
-      } else {
-        c = modeCtx<App>(p.roots[r.root]);
-        expand<App>(p, c, r, w);
-        have = true;
-      }
-    }
-    if (have) {
-      const KdNodeD leaf = p.sv.nodes[r.node];
-      const LeafTri ref = p.sv.refs[leaf.offset + uint32_t(r.cursor)];
-      const TriS ti = triSetup(c, ref);
-      tri = ti.tri;
-      classifyTri(c, w, ti, L, nl);  // kClip, as found by the trace
-      CountSink cs;
-      cs.col = stageCol;
-      Ln Lc[5];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) Lc[k] = L[k];
-      clipTri(c, w.b, Lc, nl, cs, cnt.v[sFive]);
-      commit = cs.hitArea >= c.minArea;
-      recs0 = cs.recs0;
-      staged = cs.overflow ? -1 : cs.staged;
-      slots = commit ? cs.recs0 + (c.anyHit() ? 0 : cs.recs1) : 1;
-      const int old = atomicAdd(&p.live[r.root], slots - 1);
-      if (old + slots - 1 > p.budget) {
-        killRoot(p, r.root);
-        liveSub(p, r.root, slots);
-        slots = 0;
-      } else {
-        emit = true;
-        if (slots == 0 && old == 1) rootDone(p, r.root);
-      }
-    }
-    const int slot = waveAppend(&p.st->count[nxt], slots);
-    if (slots > 0 && (unsigned long long)(slot + slots) > p.capacity) {
-      p.st->overflow = 1;
-      emit = false;
-    }
-    if (emit) {
-      Rec b = r;
-      b.cursor = r.cursor + 1;
-      Rec* dst = p.tq[nxt] + slot;
-      if (!commit) {
-        dst[0] = b;
-      } else {
-        cnt.v[sSplits]++;
-        EmitSink<App> es;
-        es.p = &p;
-        es.c = &c;
-        es.parent = &w.b;
-        es.base = &b;
-        es.dst = dst;
-        es.k0 = 0;
-        es.k1 = recs0;
-        es.t = tri;
-        es.cnt = &cnt;
-        if (staged >= 0) {  // replay the counting pass's pieces in their order
-          for (int k = 0; k < staged; ++k) {
-            const float* rd = stageCol + k * kStageWords * kBlock;
-            Pg<6> q;
-#pragma unroll
-            for (int v = 0; v < 5; ++v) {
-              q.x[v] = rd[v * kBlock];
-              q.y[v] = rd[(5 + v) * kBlock];
-            }
-            q.x[5] = q.y[5] = 0;
-            const int tag = __float_as_int(rd[10 * kBlock]);
-            q.n = tag & 0xff;
-            es.push((tag >> 8) & 1, q, ((tag >> 9) & 1) != 0);
-          }
-        } else {
-          uint32_t dummyFive = 0;
-          clipTri(c, w.b, L, nl, es, dummyFive);
-        }
-      }
+// Clips the pending triangle out of each calling lane's sub-beam r (lanes with
+// `valid`; all 64 lanes call it): the pieces it leaves become records, written
+// where alloc(slots) says for each lane (null: no room, which alloc has dealt
+// with).
+template <int App, class Alloc>
+__device__ __forceinline__ void clipChunk(const Params& p, bool valid, const Rec& r, float* stageCol, Cnt& cnt,
+                                          Alloc alloc) {
+  int slots = 0;
+  bool have = false, emit = false, commit = false;
+  Work w;
+  Ctx c;
+  Ln L[5];
+  int nl = 0;
+  int recs0 = 0;
+  int staged = -1;  // pieces kept in LDS by the counting pass (-1: clip again)
+  int tri = -1;
+  if (valid) {
+    if (p.state[r.root] == kKilled) {
+      liveSub(p, r.root, 1);
+    } else {
+      c = modeCtx<App>(p.roots[r.root]);
+      expand<App>(p, c, r, w);
+      have = true;
     }
   }
-  flushCnt(p, cnt);
-  // The last workgroup to finish schedules the next round: the last of each
-  // group of workgroups counts its group done, the last group schedules.
+  if (have) {
+    const KdNodeD leaf = p.sv.nodes[r.node];
+    const LeafTri ref = p.sv.refs[leaf.offset + uint32_t(r.cursor)];
+    const TriS ti = triSetup(c, ref);
+    tri = ti.tri;
+    classifyTri(c, w, ti, L, nl);  // kClip, as found by the trace
+    CountSink cs;
+    cs.col = stageCol;
+    Ln Lc[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) Lc[k] = L[k];
+    uint32_t five = 0;  // counted apart: a pointer into cnt would keep it out of registers
+    clipTri(c, w.b, Lc, nl, cs, five);
+    cnt.v[sFive] += five;
+    commit = cs.hitArea >= c.minArea;
+    recs0 = cs.recs0;
+    staged = cs.overflow ? -1 : cs.staged;
+    slots = commit ? cs.recs0 + (c.anyHit() ? 0 : cs.recs1) : 1;
+    const int old = atomicAdd(&p.live[r.root], slots - 1);
+    if (old + slots - 1 > p.budget) {
+      killRoot(p, r.root);
+      liveSub(p, r.root, slots);
+      slots = 0;
+    } else {
+      emit = true;
+      if (slots == 0 && old == 1) rootDone(p, r.root);
+    }
+  }
+  Rec* const dst = alloc(slots);
+  if (!emit || (slots > 0 && !dst)) return;
+  Rec b = r;
+  b.cursor = r.cursor + 1;
+  if (!commit) {
+    dst[0] = b;
+    return;
+  }
+  cnt.v[sSplits]++;
+  EmitSink<App> es;
+  es.p = &p;
+  es.c = &c;
+  es.parent = &w.b;
+  es.base = &b;
+  es.dst = dst;
+  es.k0 = 0;
+  es.k1 = recs0;
+  es.t = tri;
+  Cnt emitted;
+  emitted.zero();
+  es.cnt = &emitted;
+  if (staged >= 0) {  // replay the counting pass's pieces in their order
+    for (int k = 0; k < staged; ++k) {
+      const float* rd = stageCol + k * kStageWords * kBlock;
+      Pg<6> q;
+#pragma unroll
+      for (int v = 0; v < 5; ++v) {
+        q.x[v] = rd[v * kBlock];
+        q.y[v] = rd[(5 + v) * kBlock];
+      }
+      q.x[5] = q.y[5] = 0;
+      const int tag = __float_as_int(rd[10 * kBlock]);
+      q.n = tag & 0xff;
+      es.push((tag >> 8) & 1, q, ((tag >> 9) & 1) != 0);
+    }
+  } else {
+    uint32_t dummyFive = 0;
+    clipTri(c, w.b, L, nl, es, dummyFive);
+  }
+  cnt.v[sFive] += emitted.v[sFive];
+  cnt.v[sHits] += emitted.v[sHits];
+  cnt.v[sBeams] += emitted.v[sBeams];
+  cnt.dropped += emitted.dropped;
+}
+
+// The last workgroup of a round's last launch to get here schedules the next
+// round: the last of each group of workgroups counts its group done, the last
+// group schedules. All threads of every workgroup call it once.
+__device__ __forceinline__ void finishRound(const Params& p, int cur) {
   __syncthreads();
   if (threadIdx.x == 0) {
     const int G = int(gridDim.x), g = int(blockIdx.x) % kXcds;
@@ -1835,6 +1877,269 @@ __global__ void __launch_bounds__(kBlock) SPLIT_OCCUPANCY splitKernel(Params p, 
   }
 }
 
+template <int App>
+__global__ void __launch_bounds__(kBlock) SPLIT_OCCUPANCY splitKernel(Params p, int cur) {
+  Cnt cnt;
+  cnt.zero();
+  __shared__ float stageLds[kStageSlots * kStageWords * kBlock];
+  const int n = int(min((unsigned long long)p.st->splitCount, p.capacity));
+  const int nxt = cur ^ 1;
+  const Deal dl = dealOf();
+  bool first = true, exhausted = false;
+  while (n > 0 && !exhausted) {  // an empty round skips to the scheduling below
+    const int base = nextChunk(dl, &p.st->head[kHeadSplit], kWave, n, first, exhausted);
+    if (base >= n) break;
+    const int i = base + lane();
+    Rec r;
+    if (i < n) r = p.sq[i];
+    clipChunk<App>(p, i < n, r, stageLds + threadIdx.x, cnt, [&](int slots) -> Rec* {
+      const int slot = waveAppend(&p.st->count[nxt], slots);
+      return roomAt(p, nxt, slot, slots, r.root);
+    });
+  }
+  flushCnt(p, cnt);
+  finishRound(p, cur);
+}
+
+// The exact Lambert integral of an unoccluded piece (polygonFormFactorG,
+// soft_core.h:18-33), summed per root in 2^-60 fixed point; guarded: in double
+// throughout. Pieces are integrated 64 at a time, apart from the trace, so that
+// this double-precision code raises neither its registers nor its divergence.
+template <bool Guarded>
+__device__ __forceinline__ void shadeOne(const Params& p, const ShadeRec& sr) {
+  const RootQ& R = p.roots[sr.root];
+  double G;
+  if (Guarded) {
+    const Plane& pl = R.plane;
+    D3 P[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double qx = sr.qx[k], qy = sr.qy[k];
+      P[k] = D3{(double(pl.p0.x) + double(pl.u.x) * qx) + double(pl.v.x) * qy,
+                (double(pl.p0.y) + double(pl.u.y) * qx) + double(pl.v.y) * qy,
+                (double(pl.p0.z) + double(pl.u.z) * qx) + double(pl.v.z) * qy};
+    }
+    const D3 xd{double(R.x.x) + double(R.xlo.x), double(R.x.y) + double(R.xlo.y), double(R.x.z) + double(R.xlo.z)};
+    G = formFactorD(xd, D3{R.ns.x, R.ns.y, R.ns.z}, P, sr.n);
+  } else {
+    F3 P[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) P[k] = R.plane.point(sr.qx[k], sr.qy[k]);
+    G = double(formFactor(R.x, R.ns, P, sr.n));
+  }
+  atomicAdd(&p.gFx[sr.root], (unsigned long long)rint(G * pow2(60)));
+}
+
+// The pieces queued this round.
+__global__ void __launch_bounds__(kBlock) shadeKernel(Params p) {
+  const int n = int(min((unsigned long long)p.st->shadeCount, p.capacity));
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    const ShadeRec sr = p.shq[i];
+    if (p.pixXlo)
+      shadeOne<true>(p, sr);
+    else
+      shadeOne<false>(p, sr);
+  }
+}
+
+// ------------------------------------------------------ trace and split fused
+// One launch that takes the records of a round's queue to their ends, or near
+// them: every wave traces its share 64 lanes at a time, keeps the clips it
+// meets, the records they leave and the pieces to integrate in buffers of its
+// own (Params::ws) and goes on until those and the round's queue are empty.
+//   phase A traces; its unfinished beams go back on the stack as records when
+//           it stops, so that the phases' registers do not add up;
+//   phase B clips, once enough clips wait, or once lanes idle for want of work
+//           and a clip has waited kClipWait leaf visits;
+//   phase C (exact soft shadows) integrates.
+// Waves never wait for each other. With the round's queue empty a wave goes on
+// for kLateSteps leaf visits and then hands its records to the next round,
+// which deals them evenly to all waves: a beam alone in its wave takes a third
+// of the time a step takes among 34 others, and a heavy root's beams spread
+// over the device. What a stack cannot hold goes to the next round's queue too.
+// Measured against rounds of a trace and a split launch alone: primary and
+// point shadows of the building at 1024 x 1024 19.7 -> 6.9 ms, soft shadows of
+// the conference hall at 501 x 377 19.3 -> 8.6 ms and of the room at 48 x 48 1.04
+// -> 0.56 ms. 24 leaf visits (12 and 8 took 1 to 7% longer) and a wait of 4 (2
+// and 1: 5 to 15% longer) were the best of those tried.
+// While a round's queue fills the device (kDenseRecs), those rounds are faster:
+// their kernels hold three waves per SIMD, this one two (the plant at 512 x 512
+// 111 ms, 132 ms fused throughout; runPassApp).
+constexpr int kWsTrace = 1024, kWsClip = 256;  // records of a wave's two stacks
+constexpr int kWsShade = 512;                  // pieces of its integral buffer
+constexpr int kWsBytes = (kWsTrace + kWsClip) * int(sizeof(Rec)) + kWsShade * int(sizeof(ShadeRec));
+#ifndef BTG_CLIP_WAIT
+#define BTG_CLIP_WAIT 4
+#endif
+#ifndef BTG_LATE_STEPS
+#define BTG_LATE_STEPS 24
+#endif
+constexpr int kClipWait = BTG_CLIP_WAIT, kLateSteps = BTG_LATE_STEPS;
+constexpr int kTraceWords = kPathLevels + kMbox + kBoundWords, kSplitWords = kStageSlots * kStageWords;
+constexpr int kWaveWords = kTraceWords > kSplitWords ? kTraceWords : kSplitWords;
+
+template <int App>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) waveKernel(Params p, int cur) {
+  // the phases' LDS columns overlay each other: no lane holds a beam while its wave clips
+  __shared__ uint32_t lds[kWaveWords * kBlock];
+  __shared__ int shadeCounts[kBlock / kWave];
+  const int n = int(min((unsigned long long)p.st->count[cur], p.capacity));
+  const int nxt = cur ^ 1;
+  const bool shade = isSoft(App) && p.exact;
+  if (shade) {  // pieces of roots whose beams miss the scene, queued at admission
+    const int m = int(min((unsigned long long)p.st->shadeCount, p.capacity));
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < m; i += gridDim.x * kBlock)
+      shadeOne<App == kSoftG>(p, p.shq[i]);
+  }
+  if (n > 0) {
+    Cnt cnt;
+    cnt.zero();
+    const Deal dl = dealOf();
+    char* const ws = p.ws + size_t(dl.wave) * kWsBytes;
+    Rec* const ts = reinterpret_cast<Rec*>(ws);
+    Rec* const cs = ts + kWsTrace;
+    int* const shN = &shadeCounts[threadIdx.x / kWave];
+    *shN = 0;
+    const WaveShade wsh{shade ? reinterpret_cast<ShadeRec*>(cs + kWsClip) : nullptr, shN};
+    int tsN = 0, csN = 0, late = 0;
+    // short queues are dealt evenly, a few records per wave, long ones by 64
+    const int share = min((n + dl.waves - 1) / dl.waves, kWave), statics = share * dl.waves;
+    bool first = true, exhausted = false;
+    for (;;) {
+      {  // phase A
+        const Path path{lds + threadIdx.x};
+        int32_t* const mboxLds = reinterpret_cast<int32_t*>(lds + kPathLevels * kBlock);
+        float* const bounds = reinterpret_cast<float*>(lds + (kPathLevels + kMbox) * kBlock) + threadIdx.x;
+        bool active = false;
+        int waited = 0;
+        // set, not left undefined: an undefined value may be carried over from the
+        // phase before, and the phases' registers would add up
+        Rec r{};
+        Work w{};
+        Ctx c{};
+        Stepper ss;
+        ss.phase = kDescend;
+        ss.sd.nIn.x = ss.sd.nIn.y = ss.sd.nIn.z = ss.sd.nOut.x = ss.sd.nOut.y = ss.sd.nOut.z = 0;
+        ss.kn.split = 0;
+        ss.kn.data = ss.kn.offset = ss.leafOffset = ss.leafCount = ss.ancBase = 0;
+        ss.validFrom = 0;
+        ss.slow = false;
+        for (;;) {
+          const uint64_t idle = __ballot(!active);
+          const int nIdle = __popcll(idle);
+          if (nIdle > 0 && (tsN > 0 || !exhausted)) {
+            const int rank = rankBelow(idle), take = min(nIdle, tsN);
+            bool got = false;
+            if (!active && rank < take) {
+              r = ts[tsN - 1 - rank];
+              got = true;
+            }
+            tsN -= take;
+            if (take < nIdle && !exhausted) {
+              int base = 0, want = nIdle - take;
+              if (first) {
+                first = false;
+                base = dl.wave * share;
+                want = min(want, share);
+                exhausted = statics >= n;
+              } else {
+                if (lane() == 0) base = atomicAdd(&p.st->head[kHeadTrace], want);
+                base = __shfl(base, 0, kWave) + statics;
+                exhausted = base + want >= n;
+              }
+              const int i = base + (rank - take);
+              if (!active && rank >= take && rank - take < want && i < n) {
+                r = p.tq[cur][i];
+                got = true;
+              }
+            }
+            if (got) active = loadBeam<App>(p, c, r, w, ss, bounds, mboxLds);
+          }
+          if (!__any(active)) {
+            if (tsN > 0 || !exhausted) continue;
+            break;
+          }
+          if (exhausted) ++late;
+          int res = kContinue;
+          if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt, wsh);
+          const bool want = active && res == kContinue;
+          const int cr = coopTest<App>(p, c, r, w, ss, want, cnt, mboxLds, bounds);
+          if (want) res = cr;
+          if (active) {
+            if (res == kFinished) liveSub(p, r.root, 1);
+            if (res != kContinue) active = false;
+          }
+          const uint64_t splits = __ballot(res == kSplit);
+          if (res == kSplit) {
+            storeGeom(w.b, r);
+            cs[csN + rankBelow(splits)] = r;
+          }
+          csN += __popcll(splits);
+          const uint64_t busy = __ballot(active);
+          const bool starved = exhausted && tsN == 0 && __popcll(busy) < kWave;
+          if (csN > kWsClip - kWave || (csN > 0 && (!busy || (starved && ++waited >= kClipWait))) ||
+              (shade && *(volatile int*)shN > kWsShade - kWave) || late >= kLateSteps) {
+            const bool room = tsN + kWave <= kWsTrace;
+            if (active) {
+              storeGeom(w.b, r);
+              if (room)
+                ts[tsN + rankBelow(busy)] = r;
+              else
+                toQueue(p, nxt, activeAppend(&p.st->count[nxt]), r);
+            }
+            if (room) tsN += __popcll(busy);
+            break;
+          }
+        }
+      }
+      __threadfence_block();
+      while (csN > 0) {  // phase B
+        const int m = min(csN, kWave);
+        csN -= m;
+        Rec r{};
+        if (lane() < m) r = cs[csN + lane()];
+        clipChunk<App>(p, lane() < m, r, reinterpret_cast<float*>(lds) + threadIdx.x, cnt, [&](int slots) -> Rec* {
+          int x = slots;
+#pragma unroll
+          for (int o = 1; o < kWave; o <<= 1) {
+            const int y = __shfl_up(x, o, kWave);
+            if (lane() >= o) x += y;
+          }
+          const int total = __shfl(x, kWave - 1, kWave);
+          if (tsN + total <= kWsTrace) {
+            Rec* const dst = ts + tsN + (x - slots);
+            tsN += total;
+            return dst;
+          }
+          int base = 0;
+          if (lane() == 0) base = atomicAdd(&p.st->count[nxt], total);
+          base = __shfl(base, 0, kWave) + x - slots;
+          return roomAt(p, nxt, base, slots, r.root);
+        });
+      }
+      if (shade) {  // phase C
+        const int m = *(volatile int*)shN;
+        for (int k = lane(); k < m; k += kWave) shadeOne<App == kSoftG>(p, wsh.buf[k]);
+        *(volatile int*)shN = 0;
+      }
+      __threadfence_block();
+      if (late >= kLateSteps) {
+        int base = 0;
+        if (lane() == 0) base = atomicAdd(&p.st->count[nxt], tsN);
+        base = __shfl(base, 0, kWave);
+        for (int k = lane(); k < tsN; k += kWave) toQueue(p, nxt, base + k, ts[k]);
+        tsN = 0;
+      }
+      if (tsN == 0 && exhausted) break;
+      // a wave busy with its own stack learns here that the queue has run dry
+      if (!exhausted && !first)
+        exhausted = statics + *(volatile int*)&p.st->head[kHeadTrace] >= n;
+    }
+    flushCnt(p, cnt);
+  }
+  finishRound(p, cur);
+}
+
 // scheduleKernel (cuda/wavefront.cu:327-345), run by one thread after a
 // round: resets the round's counters and admits roots while their budgets fit.
 // Admits the next roots while their budgets fit in the free queue space
@@ -1845,13 +2150,13 @@ __device__ void admitNext(const Params& p) {
   const unsigned long long reserved = vs->reserved;
   const unsigned long long freeSlots = p.capacity > reserved ? p.capacity - reserved : 0;
   long long nAdmit = (long long)(p.R - vs->next);
-  const long long fit = (long long)(freeSlots / (unsigned long long)p.budget);
+  const long long fit = (long long)(freeSlots / (unsigned long long)p.reserve);
   if (fit < nAdmit) nAdmit = fit;
   if (nAdmit < 0) nAdmit = 0;
   s->admitBegin = vs->next;
   s->admitCount = int(nAdmit);
   s->next = vs->next + int(nAdmit);
-  s->reserved = reserved + (unsigned long long)nAdmit * (unsigned long long)p.budget;
+  s->reserved = reserved + (unsigned long long)nAdmit * (unsigned long long)p.reserve;
 }
 
 __device__ void scheduleNext(const Params& p, int cur) {
@@ -1902,7 +2207,6 @@ __global__ void initKernel(Params p) {
     s->done = 0;
     s->killed = 0;
     s->maxQueue = 0;
-    s->overflow = 0;
     if (p.pass == 0) s->outCount = 0;  // retry passes append to the first pass's output
     s->blocksDone = 0;
     for (int g = 0; g < kXcds; ++g) s->groupDone[g * 32] = 0;
@@ -1910,12 +2214,12 @@ __global__ void initKernel(Params p) {
     s->reserved = 0;
     s->traceItems = s->splitItems = 0;
     long long nAdmit = p.R;
-    const long long fit = (long long)(p.capacity / (unsigned long long)p.budget);
+    const long long fit = (long long)(p.capacity / (unsigned long long)p.reserve);
     if (fit < nAdmit) nAdmit = fit;
     s->admitBegin = 0;
     s->admitCount = int(nAdmit);
     s->next = int(nAdmit);
-    s->reserved = (unsigned long long)nAdmit * (unsigned long long)p.budget;
+    s->reserved = (unsigned long long)nAdmit * (unsigned long long)p.reserve;
     s->done = p.R == 0 ? 1 : 0;
   }
 }
@@ -1960,8 +2264,7 @@ __device__ bool admitPiece(const Params& p, const Ctx& c, const Pg<8>& qd, const
   r.depth = 0;
   const int slot = atomicAdd(&p.st->count[cur], 1);
   if ((unsigned long long)slot >= p.capacity) {
-    p.st->overflow = 1;
-    ao.ok = false;
+    ao.ok = false;  // the root is abandoned
     return false;
   }
   p.tq[cur][slot] = r;
@@ -2258,38 +2561,6 @@ __global__ void __launch_bounds__(kBlock) admitKernel(Params p, int cur) {
     }
   }
   flushCnt(p, cnt);
-}
-
-// The exact Lambert integral of the unoccluded pieces queued this round
-// (polygonFormFactorG, soft_core.h:18-33), summed per root in 2^-60 fixed
-// point. Kept out of the trace kernel so that its double-precision code does
-// not raise the trace kernel's register count.
-__global__ void __launch_bounds__(kBlock) shadeKernel(Params p) {
-  const int n = int(min((unsigned long long)p.st->shadeCount, p.capacity));
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    const ShadeRec sr = p.shq[i];
-    const RootQ& R = p.roots[sr.root];
-    double G;
-    if (p.pixXlo) {  // guarded: in double throughout
-      const Plane& pl = R.plane;
-      D3 P[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double qx = sr.qx[k], qy = sr.qy[k];
-        P[k] = D3{(double(pl.p0.x) + double(pl.u.x) * qx) + double(pl.v.x) * qy,
-                  (double(pl.p0.y) + double(pl.u.y) * qx) + double(pl.v.y) * qy,
-                  (double(pl.p0.z) + double(pl.u.z) * qx) + double(pl.v.z) * qy};
-      }
-      const D3 xd{double(R.x.x) + double(R.xlo.x), double(R.x.y) + double(R.xlo.y), double(R.x.z) + double(R.xlo.z)};
-      G = formFactorD(xd, D3{R.ns.x, R.ns.y, R.ns.z}, P, sr.n);
-    } else {
-      F3 P[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) P[k] = R.plane.point(sr.qx[k], sr.qy[k]);
-      G = double(formFactor(R.x, R.ns, P, sr.n));
-    }
-    atomicAdd(&p.gFx[sr.root], (unsigned long long)rint(G * pow2(60)));
-  }
 }
 
 // finalizeSoftKernel (cuda/wavefront.cu:539-561) with the exact sums:
@@ -2735,7 +3006,7 @@ class Engine {
   // scene storage
   void* sceneMem[7] = {};
   // engine buffers (grown on demand)
-  DevBuf tq0, tq1, sq, roots, live, state, epoch, missFx, gFx, stats, st, out, outRoot, outTag, list, listCount;
+  DevBuf tq0, tq1, sq, ws, roots, live, state, epoch, missFx, gFx, stats, st, out, outRoot, outTag, list, listCount;
   DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, prim, retry, cycles, shq, jobs;
   // FP64 soft shadows: hit leaf reference per pixel; counters and cell lists;
   // the tracers' arrays; the jobs' double cameras; per-pixel fixed-point sums
@@ -2790,7 +3061,7 @@ class Engine {
     return 0;
   }
   ~Engine() {
-    DevBuf* all[] = {&tq0, &tq1, &sq, &roots, &live, &state, &epoch, &missFx, &gFx, &stats, &st, &out,
+    DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &stats, &st, &out,
                      &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterRows, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
     for (DevBuf* b : all)
       if (b->ptr) (void)hipFree(b->ptr);
@@ -2837,6 +3108,7 @@ int prepare(Engine& e, int app, int R, int budget, Params& p, std::string& err) 
   p.R = R;
   p.rootList = nullptr;
   p.budget = budget;
+  p.reserve = budget;
   p.capacity = (unsigned long long)cap;
   p.tq[0] = static_cast<Rec*>(e.tq0.ptr);
   p.tq[1] = static_cast<Rec*>(e.tq1.ptr);
@@ -2890,9 +3162,22 @@ struct RoundGraphs {
   }
 };
 
+#ifndef BTG_DENSE
+#define BTG_DENSE (1 << 18)
+#endif
+// Queue records from which rounds run as separate launches: a third more than
+// the lanes that three waves per SIMD hold (half the line changes nothing, twice
+// it costs the plant 20%).
+constexpr long long kDenseRecs = BTG_DENSE;
+constexpr int kFusedCheck = 4;               // fused rounds between state read-backs, at most
+#ifndef BTG_RESERVE
+#define BTG_RESERVE 128
+#endif
+constexpr int kReserveMin = 32, kReserveMax = BTG_RESERVE;  // at least what a root is admitted with (8 sign regions, fans of 3)
+
 // Runs the rounds of one pass until the state reports done: groups of
-// roundsPerCheck rounds (admit, trace, shade, split each), then one state
-// read-back. With Options::graphs each group is captured once into a HIP
+// roundsPerCheck rounds (admit, trace, shade, split each, or admit and the
+// fused kernel), then one state read-back. With Options::graphs each group is captured once into a HIP
 // graph and replayed; the kernels read all changing state from device memory,
 // so the replays are the same launches. Per-launch timing (Options::profile)
 // brackets every launch with HIP events, which needs direct launches: events
@@ -2902,14 +3187,32 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
   const int gA = residentGrid(e, admitKernel<App>), gT = residentGrid(e, traceKernel<App>),
             gS = residentGrid(e, splitKernel<App>), gH = residentGrid(e, shadeKernel);
   const bool shade = isSoft(App) && p.exact;
-  const int k = std::max(1, e.opt.roundsPerCheck);
-  auto group = [&](int first) {
+  const int gW = residentGrid(e, waveKernel<App>);
+  if (int rc = e.ensure(e.ws, size_t(gW) * (kBlock / kWave) * kWsBytes, err)) return rc;
+  p.ws = static_cast<char*>(e.ws.ptr);
+  // A first run admits more roots at once than their budgets would fit: what
+  // matters is that the queue fills the device (with whole budgets reserved,
+  // sixteen blob and atrium jobs ran 832 rounds at 1.6 waves per SIMD, 878 ms;
+  // 640 ms with 128 records per root, which is 20 times the most that its queue
+  // ever held). Roots
+  // that find no room are abandoned and traced again with their budget reserved.
+  p.reserve = p.rootList ? p.budget : std::min(std::max(p.budget, kReserveMin), kReserveMax);
+  bool admitting = true;
+  auto group = [&](int first, int k, bool fused) {
     for (int i = 0; i < k; ++i) {
       const int cur = (first + i) & 1;
-      int ls = e.beginLaunch(0);
-      admitKernel<App><<<gA, kBlock, 0, e.stream>>>(p, cur);
-      e.endLaunch(ls);
+      int ls;
+      if (admitting) {
+        ls = e.beginLaunch(0);
+        admitKernel<App><<<gA, kBlock, 0, e.stream>>>(p, cur);
+        e.endLaunch(ls);
+      }
       ls = e.beginLaunch(1);
+      if (fused) {
+        waveKernel<App><<<gW, kBlock, 0, e.stream>>>(p, cur);
+        e.endLaunch(ls);
+        continue;
+      }
       traceKernel<App><<<gT, kBlock, 0, e.stream>>>(p, cur);
       e.endLaunch(ls);
       if (shade) {
@@ -2926,13 +3229,19 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
   BTG_TRY(hipGetLastError());
   RoundGraphs gr;
   const bool graphs = e.opt.graphs && !e.opt.profile;
+  // records of the next round's queue: at first, one per root that is admitted
+  long long queued = std::min<long long>(p.R, (long long)(p.capacity / (unsigned long long)p.reserve));
   int rounds = 0;
   for (;;) {
     const int par = rounds & 1;
-    if (graphs) {
+    const bool fused = queued < kDenseRecs;
+    // a queue not far above the line is looked at again soon: it may be shrinking
+    const int most = fused ? kFusedCheck : (queued < 8 * kDenseRecs ? 2 : e.opt.roundsPerCheck);
+    const int k = std::max(1, std::min(e.opt.roundsPerCheck, most));
+    if (graphs && k == e.opt.roundsPerCheck && !fused) {  // shorter groups are launched directly
       if (!gr.exec[par]) {
         BTG_TRY(hipStreamBeginCapture(e.stream, hipStreamCaptureModeThreadLocal));
-        group(par);
+        group(par, k, false);
         hipGraph_t g = nullptr;
         const hipError_t ce = hipStreamEndCapture(e.stream, &g);
         const hipError_t ie = ce == hipSuccess ? hipGraphInstantiate(&gr.exec[par], g, nullptr, nullptr, 0) : ce;
@@ -2941,17 +3250,16 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
       }
       BTG_TRY(hipGraphLaunch(gr.exec[par], e.stream));
     } else {
-      group(rounds);
+      group(rounds, k, fused);
     }
     rounds += k;
     BTG_TRY(hipGetLastError());
     BTG_TRY(hipMemcpyAsync(e.hostState, p.st, sizeof(WState), hipMemcpyDeviceToHost, e.stream));
     BTG_TRY(hipStreamSynchronize(e.stream));
-    if (e.hostState->overflow) {
-      err = "sub-beam queue overflow (capacity " + std::to_string(e.opt.capacity) + ")";
-      return BTG_ERR_LIMIT_CODE;
-    }
     if (e.hostState->done) break;
+    queued = (long long)e.hostState->count[rounds & 1] + e.hostState->admitCount;
+    // no root left to admit (a captured group keeps its admit launches, which find nothing)
+    if (e.hostState->next >= p.R && e.hostState->admitCount == 0) admitting = false;
     if (rounds > 200000) {
       err = "wavefront engine did not finish";
       return BTG_ERR_LIMIT_CODE;
@@ -3014,7 +3322,8 @@ int runAll(Engine& e, Params& p, int baseBudget, RunInfo& info, Finalize finaliz
     BTG_TRY(hipMemcpyAsync(&nk, e.listCount.ptr, 4, hipMemcpyDeviceToHost, e.stream));
     BTG_TRY(hipStreamSynchronize(e.stream));
     if (nk == 0) break;
-    if ((unsigned long long)budget >= p.capacity) {
+    // (after a first run that reserved less than the budget, the budget itself is still to be tried)
+    if ((unsigned long long)budget >= p.capacity && p.reserve >= budget) {
       err = "a root needs more sub-beams than the queue capacity (" + std::to_string(p.capacity) + ")";
       return BTG_ERR_LIMIT_CODE;
     }
@@ -3031,6 +3340,7 @@ int runAll(Engine& e, Params& p, int baseBudget, RunInfo& info, Finalize finaliz
     info.retries++;
     if ((rc = runPass(e, q, info, err))) return rc;
     if ((rc = finalize(q))) return rc;
+    p.reserve = q.reserve;
     p.pass = q.pass;
     p.rootList = q.rootList;
     p.R = q.R;
@@ -3845,10 +4155,6 @@ int openCollect(OpenPass* op, std::vector<int>& completed, std::vector<int>& kil
   completed.clear();
   killed.clear();
   BTG_TRY(hipEventSynchronize(op->stepDone));
-  if (e.hostState->overflow) {
-    err = "sub-beam queue overflow in an open pass";
-    return BTG_ERR_LIMIT_CODE;
-  }
   for (int j = 0; j < int(op->jobs.size()); ++j)
     if (!op->finished[size_t(j)] && op->jobLeftHost[j] == 0) completed.push_back(j);
   if (completed.empty()) return 0;
