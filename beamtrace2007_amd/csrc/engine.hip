@@ -2777,9 +2777,15 @@ constexpr int kFp64Waves = BTG_FP64_WAVES;
 
 // Triangle tests and kd steps a level-0 or level-1 cell may take before it is
 // split into finer cells (build knob BTG_FP64_WORK_CAP): bounds the time one
-// lane spends on one task, which sets the pass's tail.
+// lane spends on one task, which sets the levels' tails: a unit takes about
+// 50 us in a wave whose lanes all do different things, so at 2048 each level ran
+// for at least 100 ms. Measured at 2048 / 1024 / 512 / 384 / 256 / 128 (ms):
+// six conference jobs of sides 64 to 96 319 / - / 214 / 214 / 243 / 303, the plant
+// at 160 x 160 828 / - / 648 / 628 / 590 / 562, the room at 48 to 64 3.3 / - / 3.3 /
+// 3.3 / 4.6 / 6.3: below 384 the cells' repeated set-up costs the cheap scenes more
+// than the shorter tail gives them.
 #ifndef BTG_FP64_WORK_CAP
-#define BTG_FP64_WORK_CAP 2048
+#define BTG_FP64_WORK_CAP 384
 #endif
 constexpr uint32_t kFp64WorkCap = BTG_FP64_WORK_CAP;
 // Beams and work items of a level-1 cell's pools (build knob BTG_FP64_POOL1).
@@ -3669,7 +3675,8 @@ int softFp64(Engine& e, Params& p, size_t np, std::string& err) {
   const size_t cus = size_t(std::max(e.cus, 1)), maxBlocks = cus * 4 * kFp64Waves;
   const size_t blocks0 = std::min((np + 63) / 64, maxBlocks);
   const size_t blocks1 = std::min((16 * np + 63) / 64, maxBlocks);
-  const size_t blocks2 = std::min((256 * np + 63) / 64, cus);
+  // every level fills the device's SIMDs (level 2 on one wave per CU took 1.35 times as long on the plant)
+  const size_t blocks2 = std::min((256 * np + 63) / 64, maxBlocks);
   const size_t cap2 = std::min<size_t>(16 * np, size_t(1) << 24);  // level-2 entries
   int rc;
   if ((rc = e.ensure(e.fpMem, std::max({blocks0 * kBlock0, blocks1 * kBlock1, blocks2 * kBlock2}), err)) ||
