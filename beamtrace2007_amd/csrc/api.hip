@@ -23,7 +23,7 @@ struct btg_ctx {
 };
 
 struct btg_polys {
-  std::vector<btg::OutPoly> v;
+  btg::PolyList v;
 };
 
 namespace {
@@ -507,56 +507,6 @@ void btg_polys_free(btg_polys* p) { delete p; }
 
 }  // extern "C"
 
-namespace {
-
-bool polyLess(const btg::OutPoly& a, const btg::OutPoly& b) {
-  if (a.tri != b.tri) return a.tri < b.tri;
-  if (a.n != b.n) return a.n < b.n;
-  for (int k = 0; k < a.n; ++k) {
-    if (a.x[k] != b.x[k]) return a.x[k] < b.x[k];
-    if (a.y[k] != b.y[k]) return a.y[k] < b.y[k];
-  }
-  return a.area < b.area;
-}
-
-// The canonical order of a polygon list, sorted on up to 8 threads: parts
-// sorted on their own threads, then merged pairwise level by level. The order
-// is total on distinct polygons and equal polygons are identical bytes, so
-// the list equals a single std::sort's.
-void sortCanonical(std::vector<btg::OutPoly>& v) {
-  const size_t n = v.size();
-  const unsigned hw = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-  size_t parts = 1;
-  while (parts * 2 <= hw) parts *= 2;
-  if (n < 65536 || parts < 2) {
-    std::sort(v.begin(), v.end(), polyLess);
-    return;
-  }
-  std::vector<size_t> b(parts + 1);
-  for (size_t i = 0; i <= parts; ++i) b[i] = n * i / parts;
-  auto run = [&](auto fn, size_t count) {
-    std::vector<std::thread> th;
-    for (size_t i = 1; i < count; ++i) {
-      try {
-        th.emplace_back(fn, i);
-      } catch (const std::system_error&) {
-        fn(i);  // no thread to spare: this part on the calling thread
-      }
-    }
-    fn(size_t(0));
-    for (auto& t : th) t.join();
-  };
-  run([&](size_t i) { std::sort(v.begin() + long(b[i]), v.begin() + long(b[i + 1]), polyLess); }, parts);
-  for (size_t w = 1; w < parts; w *= 2)
-    run([&](size_t k) {
-      const size_t i = k * 2 * w;
-      std::inplace_merge(v.begin() + long(b[i]), v.begin() + long(b[i + w]), v.begin() + long(b[std::min(i + 2 * w, parts)]),
-                         polyLess);
-    }, parts / (2 * w));
-}
-
-}  // namespace
-
 extern "C" {
 
 int btg_primary(btg_ctx* ctx, const btg_camera* cam, int cull, int tile, int canonical, btg_polys** out,
@@ -568,12 +518,11 @@ int btg_primary(btg_ctx* ctx, const btg_camera* cam, int cull, int tile, int can
   try {
     btg_polys* P = new btg_polys();
     btg::RunInfo ri;
-    const int rc = btg::enginePrimary(ctx->engine, camOf(*cam), cull != 0, tile, P->v, ri, ctx->err);
+    const int rc = btg::enginePrimary(ctx->engine, camOf(*cam), cull != 0, tile, canonical != 0, P->v, ri, ctx->err);
     if (rc) {
       delete P;
       return rc;
     }
-    if (canonical) sortCanonical(P->v);
     *out = P;
     fillInfo(ri, now() - t0, info);
     if (info) info->stats.hits = uint64_t(P->v.size());
@@ -639,12 +588,11 @@ int btg_point(btg_ctx* ctx, const btg_camera* cam, const btg_poly* prim, int64_t
     btg_polys* P = new btg_polys();
     btg::RunInfo ri;
     const int rc = btg::enginePoint(ctx->engine, camOf(*cam), reinterpret_cast<const btg::OutPoly*>(prim), numPrim,
-                                    btg::f3(light3[0], light3[1], light3[2]), P->v, ri, ctx->err);
+                                    btg::f3(light3[0], light3[1], light3[2]), canonical != 0, P->v, ri, ctx->err);
     if (rc) {
       delete P;
       return rc;
     }
-    if (canonical) sortCanonical(P->v);
     *out = P;
     fillInfo(ri, now() - t0, info);
     return BTG_OK;
@@ -917,23 +865,11 @@ void pointLoop(btg_server* s) {
       polys = new btg_polys();
       btg::RunInfo ri, ri2;
       const btg::HostCam cam = camOf(r->req.cam);
-      rc = btg::enginePrimary(s->pointEngine, cam, false, 16, hits->v, ri, err);
-      if (!rc) {
-        // the point pass's output set does not depend on the order of its
-        // roots, so it runs on the device's order while the hits are sorted
-        std::vector<btg::OutPoly> roots = hits->v;
-        std::thread sorter([&] { sortCanonical(hits->v); });
-        try {
-          rc = btg::enginePoint(s->pointEngine, cam, roots.data(), int64_t(roots.size()),
-                                btg::f3(r->req.pointLight[0], r->req.pointLight[1], r->req.pointLight[2]),
-                                polys->v, ri2, err);
-        } catch (...) {
-          sorter.join();
-          throw;
-        }
-        sorter.join();
-      }
-      if (!rc) sortCanonical(polys->v);
+      rc = btg::enginePrimary(s->pointEngine, cam, false, 16, true, hits->v, ri, err);
+      if (!rc)
+        rc = btg::enginePoint(s->pointEngine, cam, hits->v.data(), int64_t(hits->v.size()),
+                              btg::f3(r->req.pointLight[0], r->req.pointLight[1], r->req.pointLight[2]), true, polys->v,
+                              ri2, err);
     } catch (const std::bad_alloc&) {
       rc = BTG_ERR_MEMORY;
       err = "host allocation failed";

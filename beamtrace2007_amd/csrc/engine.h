@@ -5,7 +5,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "beam_dev.h"
@@ -109,6 +112,24 @@ struct OutPoly {
 };
 static_assert(sizeof(OutPoly) == 44, "polygon layout");
 
+// A polygon list whose storage is not cleared before it is written.
+template <class T>
+struct NoInit : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = NoInit<U>;
+  };
+  template <class U>
+  void construct(U* p) noexcept {
+    ::new (static_cast<void*>(p)) U;
+  }
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new (static_cast<void*>(p)) U(std::forward<A>(a)...);
+  }
+};
+using PolyList = std::vector<OutPoly, NoInit<OutPoly>>;
+
 class Engine;
 
 // rasterize (src/render/render.cpp:49-95) on the device, one sample at each
@@ -191,11 +212,12 @@ int openJobs(const OpenPass* op);
 bool openIdle(const OpenPass* op);
 int openReset(OpenPass* op, std::string& err);
 
-// Primary visibility, one root per tile: hit polygons.
-int enginePrimary(Engine* e, const HostCam& cam, bool cull, int tile, std::vector<OutPoly>& out, RunInfo& info,
+// Primary visibility, one root per tile: hit polygons (canonical: in the
+// reference's canonical order, else the device's).
+int enginePrimary(Engine* e, const HostCam& cam, bool cull, int tile, bool canonical, PolyList& out, RunInfo& info,
                   std::string& err);
 // Point shadows for primary hit polygons.
 int enginePoint(Engine* e, const HostCam& cam, const OutPoly* prim, int64_t nPrim, F3 light,
-                std::vector<OutPoly>& out, RunInfo& info, std::string& err);
+                bool canonical, PolyList& out, RunInfo& info, std::string& err);
 
 }  // namespace btg

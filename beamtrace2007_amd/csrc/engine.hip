@@ -3014,6 +3014,7 @@ class Engine {
   // engine buffers (grown on demand)
   DevBuf tq0, tq1, sq, ws, roots, live, state, epoch, missFx, gFx, stats, st, out, outRoot, outTag, list, listCount;
   DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, prim, retry, cycles, shq, jobs;
+  DevBuf valid, order, sorted;  // polygon lists on their way out: after retries, two orders, in canonical order
   // FP64 soft shadows: hit leaf reference per pixel; counters and cell lists;
   // the tracers' arrays; the jobs' double cameras; per-pixel fixed-point sums
   DevBuf pixRef, fpList, fpMem, camD, fpSum;
@@ -3068,7 +3069,7 @@ class Engine {
   }
   ~Engine() {
     DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &stats, &st, &out,
-                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterRows, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
+                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterRows, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &valid, &order, &sorted, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
     for (DevBuf* b : all)
       if (b->ptr) (void)hipFree(b->ptr);
     for (void* m : sceneMem)
@@ -4195,22 +4196,129 @@ int openCollect(OpenPass* op, std::vector<int>& completed, std::vector<int>& kil
 
 namespace {
 
-// Downloads the polygons whose tag equals their root's last pass.
-int downloadPolys(Engine& e, int R, std::vector<OutPoly>& polys, std::string& err) {
-  const int n = std::min(e.hostState->outCount, int(e.out.bytes / sizeof(OutPoly)));
-  std::vector<OutPoly> out(static_cast<size_t>(std::max(n, 0)));
-  std::vector<int> root(out.size()), tag(out.size()), epoch(static_cast<size_t>(R));
-  if (n > 0) {
-    BTG_TRY(hipMemcpyAsync(out.data(), e.out.ptr, sizeof(OutPoly) * size_t(n), hipMemcpyDeviceToHost, e.stream));
-    BTG_TRY(hipMemcpyAsync(root.data(), e.outRoot.ptr, sizeof(int) * size_t(n), hipMemcpyDeviceToHost, e.stream));
-    BTG_TRY(hipMemcpyAsync(tag.data(), e.outTag.ptr, sizeof(int) * size_t(n), hipMemcpyDeviceToHost, e.stream));
+// ---------------------------------------------------------- canonical order
+// polyLess of the reference's canonical list: triangle, corner count, corners, area.
+__device__ __forceinline__ bool polyLess(const OutPoly& a, const OutPoly& b) {
+  if (a.tri != b.tri) return a.tri < b.tri;
+  if (a.n != b.n) return a.n < b.n;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (k >= a.n) break;
+    if (a.x[k] != b.x[k]) return a.x[k] < b.x[k];
+    if (a.y[k] != b.y[k]) return a.y[k] < b.y[k];
   }
-  if (R > 0) BTG_TRY(hipMemcpyAsync(epoch.data(), e.epoch.ptr, sizeof(int) * size_t(R), hipMemcpyDeviceToHost, e.stream));
-  BTG_TRY(hipStreamSynchronize(e.stream));
+  return a.area < b.area;
+}
+
+// The sort works on polygon numbers: blocks of kSortBlock put in order by
+// counting, then runs merged pairwise, every element finding its place by a
+// binary search of its sibling run. Most comparisons end at the triangle. Both
+// steps are stable, so places are distinct also for equal polygons.
+constexpr int kSortBlock = 256;
+__global__ void __launch_bounds__(kSortBlock) sortBlocks(const OutPoly* polys, int n, int* order) {
+  __shared__ int tris[kSortBlock];
+  const int base = int(blockIdx.x) * kSortBlock, i = base + int(threadIdx.x);
+  const int m = min(kSortBlock, n - base);
+  OutPoly own{};
+  if (i < n) own = polys[i];
+  tris[threadIdx.x] = own.tri;
+  __syncthreads();
+  if (i >= n) return;
+  int rank = 0;
+  for (int j = 0; j < m; ++j) {
+    const int t = tris[j];
+    bool before = t < own.tri;
+    if (t == own.tri && base + j != i) {
+      const OutPoly other = polys[base + j];
+      before = polyLess(other, own) || (base + j < i && !polyLess(own, other));
+    }
+    rank += before;
+  }
+  order[base + rank] = i;
+}
+
+__global__ void __launch_bounds__(256) mergeRuns(const OutPoly* polys, const int* in, int* out, int n, int run) {
+  const int i = int(blockIdx.x) * 256 + int(threadIdx.x);
+  if (i >= n) return;
+  const int mine = i / run, begin = mine * run;
+  const int64_t sib = int64_t(mine ^ 1) * run;
+  const int k = in[i];
+  const OutPoly own = polys[k];
+  int lo = 0;
+  if (sib < n) {
+    int hi = int(min(int64_t(run), int64_t(n) - sib));
+    const bool second = mine & 1;  // elements of the first run precede their equals
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      const OutPoly other = polys[in[sib + mid]];
+      if (second ? !polyLess(own, other) : polyLess(other, own))
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+  }
+  out[(mine & ~1) * int64_t(run) + (i - begin) + lo] = k;
+}
+
+// Polygons in the order of their numbers, one 4-byte word per thread.
+__global__ void __launch_bounds__(256) gatherPolys(const OutPoly* polys, const int* order, int n, OutPoly* dst) {
+  constexpr int kWords = int(sizeof(OutPoly) / 4);
+  const int64_t w = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (w >= int64_t(n) * kWords) return;
+  const int i = int(w / kWords), k = int(w % kWords);
+  reinterpret_cast<uint32_t*>(dst)[w] = reinterpret_cast<const uint32_t*>(polys + order[i])[k];
+}
+
+// Valid polygons of the last pass (tag == epoch[root]), compacted.
+__global__ void compactPolys(const OutPoly* polys, const int* root, const int* tag, const int* epoch, int n,
+                             OutPoly* dst, int* count) {
+  const int i = int(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n || tag[i] != epoch[root[i]]) return;
+  dst[atomicAdd(count, 1)] = polys[i];
+}
+
+// Downloads the pass's polygons; after retries (`filter`) those whose tag
+// equals their root's last pass. Canonical lists are sorted on the device:
+// primary and point shadows of the conference hall (220K and 230K polygons at
+// 640 x 481) take 21.8 ms, and 30.7 ms with the lists sorted on eight host
+// threads and their tags filtered there.
+int takePolys(Engine& e, bool filter, bool canonical, PolyList& polys, std::string& err) {
+  int n = std::max(0, std::min(e.hostState->outCount, int(e.out.bytes / sizeof(OutPoly))));
+  const OutPoly* src = static_cast<const OutPoly*>(e.out.ptr);
+  int rc;
   polys.clear();
-  polys.reserve(out.size());
-  for (int i = 0; i < n; ++i)
-    if (tag[size_t(i)] == epoch[size_t(root[size_t(i)])]) polys.push_back(out[size_t(i)]);
+  if (n == 0) return 0;
+  if (filter) {
+    if ((rc = e.ensure(e.valid, size_t(n) * sizeof(OutPoly), err)) || (rc = e.ensure(e.listCount, 4, err))) return rc;
+    clearInt<<<1, 64, 0, e.stream>>>(static_cast<int*>(e.listCount.ptr));
+    compactPolys<<<(n + 255) / 256, 256, 0, e.stream>>>(src, static_cast<const int*>(e.outRoot.ptr),
+                                                        static_cast<const int*>(e.outTag.ptr),
+                                                        static_cast<const int*>(e.epoch.ptr), n,
+                                                        static_cast<OutPoly*>(e.valid.ptr),
+                                                        static_cast<int*>(e.listCount.ptr));
+    BTG_TRY(hipGetLastError());
+    BTG_TRY(hipMemcpyAsync(&n, e.listCount.ptr, 4, hipMemcpyDeviceToHost, e.stream));
+    BTG_TRY(hipStreamSynchronize(e.stream));
+    src = static_cast<const OutPoly*>(e.valid.ptr);
+    if (n == 0) return 0;
+  }
+  if (canonical && n > 1) {
+    if ((rc = e.ensure(e.order, size_t(n) * 2 * sizeof(int), err)) ||
+        (rc = e.ensure(e.sorted, size_t(n) * sizeof(OutPoly), err)))
+      return rc;
+    int* a = static_cast<int*>(e.order.ptr);
+    int* b = a + n;
+    sortBlocks<<<(n + kSortBlock - 1) / kSortBlock, kSortBlock, 0, e.stream>>>(src, n, a);
+    for (int64_t run = kSortBlock; run < n; run *= 2, std::swap(a, b))
+      mergeRuns<<<(n + 255) / 256, 256, 0, e.stream>>>(src, a, b, n, int(run));
+    gatherPolys<<<unsigned((int64_t(n) * int64_t(sizeof(OutPoly) / 4) + 255) / 256), 256, 0, e.stream>>>(
+        src, a, n, static_cast<OutPoly*>(e.sorted.ptr));
+    BTG_TRY(hipGetLastError());
+    src = static_cast<const OutPoly*>(e.sorted.ptr);
+  }
+  polys.resize(size_t(n));
+  BTG_TRY(hipMemcpyAsync(polys.data(), src, sizeof(OutPoly) * size_t(n), hipMemcpyDeviceToHost, e.stream));
+  BTG_TRY(hipStreamSynchronize(e.stream));
   return 0;
 }
 
@@ -4227,8 +4335,8 @@ size_t outCapFor(const Engine& e, size_t want) {
 // With download = false the polygons stay on the device (e.out, filtered by
 // outTag == epoch[outRoot]) for a device-side consumer.
 template <class Setup>
-int runPolys(Engine& e, int app, int R, int budget, size_t outCap, const HostCam& cam, Setup setup,
-             std::vector<OutPoly>& polys, RunInfo& info, std::string& err, bool download = true) {
+int runPolys(Engine& e, int app, int R, int budget, size_t outCap, const HostCam& cam, Setup setup, bool canonical,
+             PolyList& polys, RunInfo& info, std::string& err, bool download = true) {
   for (;;) {
     Params p;
     int rc = prepare(e, app, R, budget, p, err);
@@ -4259,7 +4367,7 @@ int runPolys(Engine& e, int app, int R, int budget, size_t outCap, const HostCam
     ri.traceMs = ms;
     if ((rc = readStats(e, ri.stats, &ri.dropped, err))) return rc;
     e.collectLaunches(ri);
-    if (download && (rc = downloadPolys(e, R, polys, err))) return rc;
+    if (download && (rc = takePolys(e, ri.retries > 0, canonical, polys, err))) return rc;
     info = ri;
     return 0;
   }
@@ -4267,7 +4375,7 @@ int runPolys(Engine& e, int app, int R, int budget, size_t outCap, const HostCam
 
 }  // namespace
 
-int enginePrimary(Engine* e, const HostCam& cam, bool cull, int tile, std::vector<OutPoly>& out, RunInfo& info,
+int enginePrimary(Engine* e, const HostCam& cam, bool cull, int tile, bool canonical, PolyList& out, RunInfo& info,
                   std::string& err) {
   if (tile <= 0 || cam.W <= 0 || cam.H <= 0) {
     err = "tile and image size must be positive";
@@ -4280,11 +4388,11 @@ int enginePrimary(Engine* e, const HostCam& cam, bool cull, int tile, std::vecto
     p.tilesW = tilesW;
     p.cull = cull ? 1 : 0;
   };
-  return runPolys(*e, kPrimary, tilesW * tilesH, e->opt.primaryBudget, outCap, cam, setup, out, info, err);
+  return runPolys(*e, kPrimary, tilesW * tilesH, e->opt.primaryBudget, outCap, cam, setup, canonical, out, info, err);
 }
 
-int enginePoint(Engine* e, const HostCam& cam, const OutPoly* prim, int64_t nPrim, F3 light,
-                std::vector<OutPoly>& out, RunInfo& info, std::string& err) {
+int enginePoint(Engine* e, const HostCam& cam, const OutPoly* prim, int64_t nPrim, F3 light, bool canonical,
+                PolyList& out, RunInfo& info, std::string& err) {
   out.clear();
   if (nPrim <= 0) return 0;
   if (nPrim > (1LL << 30)) {
@@ -4304,7 +4412,7 @@ int enginePoint(Engine* e, const HostCam& cam, const OutPoly* prim, int64_t nPri
     p.pointLight = light;
     p.prim = static_cast<const OutPoly*>(e->prim.ptr);
   };
-  return runPolys(*e, kPoint, int(nPrim), e->opt.budget, outCap, cam, setup, out, info, err);
+  return runPolys(*e, kPoint, int(nPrim), e->opt.budget, outCap, cam, setup, canonical, out, info, err);
 }
 
 // ------------------------------------------------------------ rasterization
@@ -4511,14 +4619,6 @@ __global__ void fillByte(uint8_t* p, size_t n) {
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) p[i] = 0;
 }
 
-// Valid polygons of the last pass (tag == epoch[root]), compacted.
-__global__ void compactPolys(const OutPoly* polys, const int* root, const int* tag, const int* epoch, int n,
-                             OutPoly* dst, int* count) {
-  const int i = int(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n || tag[i] != epoch[root[i]]) return;
-  dst[atomicAdd(count, 1)] = polys[i];
-}
-
 // Device bytes of the scan scratch for n polygons: row counts (4 B each),
 // span offsets (8 B each) and tile sums (8 B per tile of kScanTile, one more).
 size_t rasterScratchBytes(int64_t n) {
@@ -4634,8 +4734,8 @@ int engineImages(Engine* e, const HostCam& cam, bool cull, int tile, const F3* l
     p.tilesW = tilesW;
     p.cull = cull ? 1 : 0;
   };
-  std::vector<OutPoly> none;
-  int rc = runPolys(*e, kPrimary, R, e->opt.primaryBudget, outCap, cam, setup, none, prim, err, false);
+  PolyList none;
+  int rc = runPolys(*e, kPrimary, R, e->opt.primaryBudget, outCap, cam, setup, false, none, prim, err, false);
   if (rc) return rc;
   const int nOut = std::min(e->hostState->outCount, int(e->out.bytes / sizeof(OutPoly)));
   auto t0 = std::chrono::steady_clock::now();
@@ -4669,7 +4769,7 @@ int engineImages(Engine* e, const HostCam& cam, bool cull, int tile, const F3* l
     p.pointLight = *light;
     p.prim = static_cast<const OutPoly*>(e->prim.ptr);
   };
-  if ((rc = runPolys(*e, kPoint, nPrim, e->opt.budget, pcap, cam, psetup, none, point, err, false))) return rc;
+  if ((rc = runPolys(*e, kPoint, nPrim, e->opt.budget, pcap, cam, psetup, false, none, point, err, false))) return rc;
   const int nShadow = std::min(e->hostState->outCount, int(e->out.bytes / sizeof(OutPoly)));
   t0 = std::chrono::steady_clock::now();
   rc = rasterDevice(*e, cam, static_cast<const OutPoly*>(e->out.ptr), static_cast<const int*>(e->outRoot.ptr),
