@@ -7,7 +7,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 #include <unordered_map>

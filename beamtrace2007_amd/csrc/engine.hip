@@ -40,13 +40,12 @@
 #include "engine.h"
 #include "kd_pred.h"
 
-// Scan scratch of the allocation-free rasterization (btg_raster_device_noalloc):
-// row counts (4 B), span offsets (8 B) and tile sums for kNoAllocMaxPolys
-// polygons, 12 MiB + 8 KiB. Every device the library runs on holds its own copy
-// until the process ends; host code reaches it only through the address
-// hipGetSymbolAddress gives on that device (noAllocScratchOn).
-static __device__ __align__(256) unsigned char noAllocScratch[btg::kNoAllocMaxPolys * 12 +
-                                                                (btg::kNoAllocMaxPolys / 1024 + 1) * 8];
+// Scratch of the allocation-free rasterization (btg_raster_device_noalloc): a
+// count and a number (4 B) for each of kNoAllocMaxPolys polygons, 4 MiB. Every
+// device the library runs on holds its own copy until the process ends; host
+// code reaches it only through the address hipGetSymbolAddress gives on that
+// device (noAllocScratchOn).
+static __device__ __align__(256) unsigned char noAllocScratch[8 + btg::kNoAllocMaxPolys * 4];
 
 namespace btg {
 
@@ -3018,7 +3017,7 @@ class Engine {
   // FP64 soft shadows: hit leaf reference per pixel; counters and cell lists;
   // the tracers' arrays; the jobs' double cameras; per-pixel fixed-point sums
   DevBuf pixRef, fpList, fpMem, camD, fpSum;
-  DevBuf rasterImg, rasterRows;  // device rasterization: image; row counts, span offsets and tile sums
+  DevBuf rasterImg, rasterTall;  // device rasterization: image; the list of the tall polygons
   void* noAllocScratch = nullptr;  // this device's static rasterization scratch (null: unavailable)
   WState* hostState = nullptr;  // pinned
   uint64_t phaseCycles[8] = {};
@@ -3069,7 +3068,7 @@ class Engine {
   }
   ~Engine() {
     DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &stats, &st, &out,
-                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterRows, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &valid, &order, &sorted, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
+                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterTall, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &valid, &order, &sorted, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
     for (DevBuf* b : all)
       if (b->ptr) (void)hipFree(b->ptr);
     for (void* m : sceneMem)
@@ -4463,124 +4462,8 @@ __device__ __forceinline__ void rasterEdges(const OutPoly& pg, float halfW, floa
   r.y1 = y1 < H - 1 ? y1 : H - 1;
 }
 
-// Per-polygon row counts are scanned into 64-bit span offsets in three
-// launches over tiles of kScanTile polygons (counts and tile sums, one block
-// scanning the tile sums, per-tile offsets). A polygon covers at most 32768
-// rows and a list at most 2^30 polygons, so 64-bit offsets cannot wrap.
-constexpr int kScanThreads = 256, kScanItems = 4, kScanTile = kScanThreads * kScanItems;
-
-// Exclusive scan of one value per thread across the block (wave64 shuffles,
-// then the waves' totals through LDS); *total receives the block's sum.
-// Every thread of the block must call it.
-__device__ __forceinline__ uint64_t blockExclusiveScan(uint64_t v, uint64_t* lds, uint64_t* total) {
-  const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6, waves = int(blockDim.x) >> 6;
-  uint64_t x = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint64_t y = __shfl_up(x, d, 64);
-    if (lane >= d) x += y;
-  }
-  if (lane == 63) lds[wave] = x;
-  __syncthreads();
-  uint64_t before = 0, all = 0;
-  for (int w = 0; w < waves; ++w) {
-    const uint64_t s = lds[w];
-    before += w < wave ? s : 0;
-    all += s;
-  }
-  __syncthreads();
-  *total = all;
-  return before + x - v;
-}
-
-// Rows a polygon covers (0 if it is filtered out): valid output of its pass
-// (tag == epoch of its root, when the epoch filter is given), a hit polygon
-// unless this is the shadow pass, 3 or 4 corners. Also each tile's row sum.
-__global__ void __launch_bounds__(kScanThreads) rasterRowsKernel(const OutPoly* polys, const int* root, const int* tag,
-                                                                 const int* epoch, int n, float halfW, float halfH,
-                                                                 int W, int H, int shadow, uint32_t* rows,
-                                                                 uint64_t* tileSum) {
-  __shared__ uint64_t lds[kScanThreads / 64];
-  const int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
-  uint64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + k;
-    if (i >= n) break;
-    const OutPoly pg = polys[i];
-    bool ok = pg.n >= 3 && pg.n <= 4 && (shadow || pg.tri >= 0);
-    if (ok && epoch) ok = tag[i] == epoch[root[i]];
-    uint32_t c = 0;
-    if (ok) {
-      RasterEdges r;
-      rasterEdges(pg, halfW, halfH, W, H, r);
-      if (r.y1 >= r.y0) c = uint32_t(r.y1 - r.y0 + 1);
-    }
-    rows[i] = c;
-    s += c;
-  }
-  uint64_t total;
-  blockExclusiveScan(s, lds, &total);
-  if (threadIdx.x == 0) tileSum[blockIdx.x] = total;
-}
-
-// Exclusive scan of the tile sums in place by one block; tileSum[tiles]
-// receives the number of spans.
-__global__ void __launch_bounds__(1024) rasterTileScanKernel(uint64_t* tileSum, int tiles) {
-  __shared__ uint64_t lds[1024 / 64];
-  uint64_t carry = 0;
-  for (int c = 0; c < tiles; c += int(blockDim.x)) {
-    const int i = c + int(threadIdx.x);
-    const uint64_t v = i < tiles ? tileSum[i] : 0;
-    uint64_t total;
-    const uint64_t ex = blockExclusiveScan(v, lds, &total);
-    if (i < tiles) tileSum[i] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) tileSum[tiles] = carry;
-}
-
-// First span of each polygon: the tile's offset plus the scan within the tile.
-__global__ void __launch_bounds__(kScanThreads) rasterOffsKernel(const uint32_t* rows, const uint64_t* tileSum, int n,
-                                                                 uint64_t* offs) {
-  __shared__ uint64_t lds[kScanThreads / 64];
-  const int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
-  uint32_t r[kScanItems];
-  uint64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    r[k] = base + k < n ? rows[base + k] : 0u;
-    s += r[k];
-  }
-  uint64_t total;
-  uint64_t ex = blockExclusiveScan(s, lds, &total) + tileSum[blockIdx.x];
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    if (base + k < n) offs[base + k] = ex;
-    ex += r[k];
-  }
-}
-
-// One (polygon, row) span per thread: the polygon is the last one whose first
-// span offset is <= the item (binary search over the exclusive scan).
-__global__ void rasterSpansKernel(const OutPoly* polys, const uint64_t* offs, int n, uint32_t total, float halfW,
-                                  float halfH, int W, int H, int shadow, int32_t* ids, uint8_t* mask) {
-  const uint32_t j = uint32_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= total) return;
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (offs[mid] <= uint64_t(j))
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  const OutPoly pg = polys[lo];
-  RasterEdges r;
-  rasterEdges(pg, halfW, halfH, W, H, r);
-  const uint64_t k = uint64_t(j) - offs[lo];
-  if (r.y1 < r.y0 || k > uint64_t(r.y1 - r.y0)) return;  // not with a consistent scan: never leave the rows
-  const int y = r.y0 + int(k);
+// The pixels [x0, x1] of row y that a polygon covers (x0 > x1: none).
+__device__ __forceinline__ void rasterSpan(const RasterEdges& r, int y, int W, int& x0, int& x1) {
   const double sy = y + 0.5;
   double xl = -1e300, xr = 1e300;
   bool empty = false;
@@ -4598,73 +4481,206 @@ __global__ void rasterSpansKernel(const OutPoly* polys, const uint64_t* offs, in
       empty = true;
     }
   }
+  x0 = 0;
+  x1 = -1;
   if (empty || xl > xr) return;
-  int x0 = toIntHost(ceil(xl - 0.5)), x1 = toIntHost(floor(xr - 0.5));
+  x0 = toIntHost(ceil(xl - 0.5));
+  x1 = toIntHost(floor(xr - 0.5));
   x0 = x0 > 0 ? x0 : 0;
   x1 = x1 < W - 1 ? x1 : W - 1;
-  const size_t row = size_t(y) * size_t(W);
-  for (int x = x0; x <= x1; ++x) {
-    if (shadow)
-      mask[row + size_t(x)] = 1;
-    else
-      atomicMax(&ids[row + size_t(x)], pg.tri);  // polygons sort by tri first: the canonical last writer
+}
+
+// Exclusive scan of one value per thread across the block (wave64 shuffles,
+// then the waves' totals through LDS); *total receives the block's sum.
+// Every thread of the block must call it.
+__device__ __forceinline__ int blockExclusiveScan(int v, int* lds, int* total) {
+  const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6, waves = int(blockDim.x) >> 6;
+  int x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) lds[wave] = x;
+  __syncthreads();
+  int before = 0, all = 0;
+  for (int w = 0; w < waves; ++w) {
+    const int s = lds[w];
+    before += w < wave ? s : 0;
+    all += s;
+  }
+  *total = all;
+  return before + x - v;
+}
+
+// Polygons to rasterize, the image, and the list of the tall ones.
+struct RasterArgs {
+  const OutPoly* polys;
+  const int *root, *tag, *epoch;  // epoch filter (epoch null: none)
+  int n;
+  float halfW, halfH;
+  int W, H, shadow;
+  int32_t* ids;
+  uint8_t* mask;
+  int* tall;                 // room for n polygon numbers
+  unsigned long long* count; // tall polygons listed; the row count of rasterCountKernel
+};
+
+// The polygon's edges and rows (0: filtered out): valid output of its pass (tag
+// == epoch of its root, when the epoch filter is given), a hit polygon unless
+// this is the shadow pass, 3 or 4 corners.
+__device__ __forceinline__ int rasterRows(const RasterArgs& a, int i, OutPoly& pg, RasterEdges& r) {
+  pg = a.polys[i];
+  bool ok = pg.n >= 3 && pg.n <= 4 && (a.shadow || pg.tri >= 0);
+  if (ok && a.epoch) ok = a.tag[i] == a.epoch[a.root[i]];
+  if (!ok) return 0;
+  rasterEdges(pg, a.halfW, a.halfH, a.W, a.H, r);
+  return r.y1 >= r.y0 ? r.y1 - r.y0 + 1 : 0;
+}
+
+__device__ __forceinline__ void rasterPixel(const RasterArgs& a, size_t at, int tri) {
+  if (a.shadow)
+    a.mask[at] = 1;
+  else
+    atomicMax(&a.ids[at], tri);  // polygons sort by tri first: the canonical last writer
+}
+
+// A workgroup takes 256 polygons and deals their rows to its threads, so that
+// one launch needs no scan over the whole list and no count on the host before
+// the next one. Polygons of more than kTallRows rows would leave a workgroup's
+// threads behind the others': they go to a list that rasterTallKernel takes a
+// row per wave, 64 pixels at a time. Bound by latency at ordinary sizes (a few
+// rows and pixels per polygon). 230K polygons of the conference hall into 512 x
+// 512 ids: 58 us for the call, 69 us in five launches with a scan over the list
+// and a read-back of its total before the last.
+constexpr int kRasterBlock = 256, kTallRows = 32, kTallSlices = 16;
+__global__ void __launch_bounds__(kRasterBlock) rasterKernel(RasterArgs a) {
+  __shared__ int offs[kRasterBlock];
+  __shared__ int waveSums[kRasterBlock / 64];
+  const int base = int(blockIdx.x) * kRasterBlock, i = base + int(threadIdx.x);
+  int rows = 0;
+  OutPoly pg;
+  RasterEdges r;
+  if (i < a.n) rows = rasterRows(a, i, pg, r);
+  if (rows > kTallRows) {
+    const uint64_t m = __ballot(1);
+    const int leader = __builtin_ctzll(m);
+    int at = 0;
+    if (lane() == leader) at = int(atomicAdd(a.count, (unsigned long long)__popcll(m)));
+    a.tall[__shfl(at, leader, kWave) + rankBelow(m)] = i;
+    rows = 0;
+  }
+  int total;
+  offs[threadIdx.x] = blockExclusiveScan(rows, waveSums, &total);
+  __syncthreads();
+  for (int j = int(threadIdx.x); j < total; j += kRasterBlock) {
+    int lo = 0, hi = kRasterBlock - 1;  // the last polygon whose first row is <= j
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (offs[mid] <= j)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    if (rasterRows(a, base + lo, pg, r) == 0) continue;  // never: its rows were counted
+    const int y = r.y0 + (j - offs[lo]);
+    int x0, x1;
+    rasterSpan(r, y, a.W, x0, x1);
+    for (int x = x0; x <= x1; ++x) rasterPixel(a, size_t(y) * size_t(a.W) + size_t(x), pg.tri);
   }
 }
 
-__global__ void fillInt(int32_t* p, size_t n, int32_t v) {
+__global__ void __launch_bounds__(kRasterBlock) rasterTallKernel(RasterArgs a) {
+  const int64_t waves = int64_t(gridDim.x) * (kRasterBlock / 64);
+  const int64_t units = int64_t(*a.count) * kTallSlices;
+  for (int64_t u = int64_t(blockIdx.x) * (kRasterBlock / 64) + threadIdx.x / 64; u < units; u += waves) {
+    OutPoly pg;
+    RasterEdges r;
+    if (rasterRows(a, a.tall[u / kTallSlices], pg, r) == 0) continue;
+    for (int y = r.y0 + int(u % kTallSlices); y <= r.y1; y += kTallSlices) {
+      int x0, x1;
+      rasterSpan(r, y, a.W, x0, x1);
+      for (int x = x0 + lane(); x <= x1; x += kWave) rasterPixel(a, size_t(y) * size_t(a.W) + size_t(x), pg.tri);
+    }
+  }
+}
+
+// The rows of all polygons together, in *a.count.
+__global__ void __launch_bounds__(kRasterBlock) rasterCountKernel(RasterArgs a) {
+  unsigned long long s = 0;
+  for (int64_t i = int64_t(blockIdx.x) * kRasterBlock + threadIdx.x; i < a.n; i += int64_t(gridDim.x) * kRasterBlock) {
+    OutPoly pg;
+    RasterEdges r;
+    s += (unsigned long long)rasterRows(a, int(i), pg, r);
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_down(s, o, kWave);
+  if (lane() == 0 && s) atomicAdd(a.count, s);
+}
+
+// The cleared image, and the list's count.
+__global__ void fillInt(int32_t* p, size_t n, int32_t v, unsigned long long* count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) p[i] = v;
 }
 
-__global__ void fillByte(uint8_t* p, size_t n) {
+__global__ void fillByte(uint8_t* p, size_t n, unsigned long long* count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) p[i] = 0;
 }
 
-// Device bytes of the scan scratch for n polygons: row counts (4 B each),
-// span offsets (8 B each) and tile sums (8 B per tile of kScanTile, one more).
-size_t rasterScratchBytes(int64_t n) {
-  const int64_t m = n > 0 ? n : 1;
-  const int64_t tiles = (m + kScanTile - 1) / kScanTile;
-  return size_t(((m * 4 + 7) & ~int64_t(7)) + m * 8 + (tiles + 1) * 8);
-}
+// Device bytes of the scratch for n polygons: the count and the list of the
+// tall ones.
+size_t rasterScratchBytes(int64_t n) { return 8 + size_t(n > 0 ? n : 1) * 4; }
 
 // Rasterizes n device polygons (epoch filter optional) into the device image
 // `img` (ids or mask, W x H) on e.stream, with `scratch` (rasterScratchBytes(n)
-// bytes of device memory) for the scan; allocates nothing. Returns after the
-// span launch is queued (the span count is read back to size it).
+// bytes of device memory); allocates nothing. Returns once the launches are
+// queued.
 int rasterInto(Engine& e, const HostCam& cam, const OutPoly* polys, const int* root, const int* tag, const int* epoch,
                int n, bool shadow, void* img, void* scratch, std::string& err) {
   const size_t np = size_t(cam.W) * size_t(cam.H);
   const int fillBlocks = int(std::min<size_t>((np + 255) / 256, 4096));
-  if (shadow)
-    fillByte<<<fillBlocks, 256, 0, e.stream>>>(static_cast<uint8_t*>(img), np);
-  else
-    fillInt<<<fillBlocks, 256, 0, e.stream>>>(static_cast<int32_t*>(img), np, -1);
+  RasterArgs a;
+  a.polys = polys;
+  a.root = root;
+  a.tag = tag;
+  a.epoch = epoch;
+  a.n = n;
+  a.halfW = cam.halfW;
+  a.halfH = cam.halfH;
+  a.W = cam.W;
+  a.H = cam.H;
+  a.shadow = shadow ? 1 : 0;
+  a.ids = static_cast<int32_t*>(img);
+  a.mask = static_cast<uint8_t*>(img);
+  a.count = static_cast<unsigned long long*>(scratch);
+  a.tall = reinterpret_cast<int*>(a.count + 1);
+  auto fill = [&] {
+    if (shadow)
+      fillByte<<<fillBlocks, 256, 0, e.stream>>>(a.mask, np, a.count);
+    else
+      fillInt<<<fillBlocks, 256, 0, e.stream>>>(a.ids, np, -1, a.count);
+  };
+  fill();
   BTG_TRY(hipGetLastError());
   if (n <= 0) return 0;
-  const int tiles = (n + kScanTile - 1) / kScanTile;
-  uint32_t* rows = static_cast<uint32_t*>(scratch);
-  uint64_t* offs = reinterpret_cast<uint64_t*>(static_cast<char*>(scratch) + ((int64_t(n) * 4 + 7) & ~int64_t(7)));
-  uint64_t* tileSum = offs + n;
-  rasterRowsKernel<<<tiles, kScanThreads, 0, e.stream>>>(polys, root, tag, epoch, n, cam.halfW, cam.halfH, cam.W,
-                                                         cam.H, shadow ? 1 : 0, rows, tileSum);
-  BTG_TRY(hipGetLastError());
-  rasterTileScanKernel<<<1, 1024, 0, e.stream>>>(tileSum, tiles);
-  BTG_TRY(hipGetLastError());
-  rasterOffsKernel<<<tiles, kScanThreads, 0, e.stream>>>(rows, tileSum, n, offs);
-  BTG_TRY(hipGetLastError());
-  uint64_t total = 0;
-  BTG_TRY(hipMemcpyAsync(&total, tileSum + tiles, 8, hipMemcpyDeviceToHost, e.stream));
-  BTG_TRY(hipStreamSynchronize(e.stream));
-  if (total > 0xffffffffull) {
-    err = "too many polygon rows to rasterize (" + std::to_string(total) + " spans; at most 2^32 - 1)";
-    return BTG_ERR_LIMIT_CODE;
-  }
-  if (total > 0) {
-    rasterSpansKernel<<<unsigned((total + 255) / 256), 256, 0, e.stream>>>(
-        polys, offs, n, uint32_t(total), cam.halfW, cam.halfH, cam.W, cam.H, shadow ? 1 : 0,
-        static_cast<int32_t*>(img), static_cast<uint8_t*>(img));
+  const int blocks = (n + kRasterBlock - 1) / kRasterBlock;
+  if (uint64_t(n) * uint64_t(cam.H) > 0xffffffffull) {  // only such a list can hold more rows than are taken
+    rasterCountKernel<<<std::min(blocks, 4096), kRasterBlock, 0, e.stream>>>(a);
     BTG_TRY(hipGetLastError());
+    unsigned long long total = 0;
+    BTG_TRY(hipMemcpyAsync(&total, a.count, 8, hipMemcpyDeviceToHost, e.stream));
+    BTG_TRY(hipStreamSynchronize(e.stream));
+    if (total > 0xffffffffull) {
+      err = "too many polygon rows to rasterize (" + std::to_string(total) + " spans; at most 2^32 - 1)";
+      return BTG_ERR_LIMIT_CODE;
+    }
+    fill();  // the count again
   }
+  rasterKernel<<<blocks, kRasterBlock, 0, e.stream>>>(a);
+  rasterTallKernel<<<std::max(e.cus, 1) * 4, kRasterBlock, 0, e.stream>>>(a);
+  BTG_TRY(hipGetLastError());
   return 0;
 }
 
@@ -4675,9 +4691,9 @@ int rasterDevice(Engine& e, const HostCam& cam, const OutPoly* polys, const int*
   const size_t np = size_t(cam.W) * size_t(cam.H);
   int rc;
   if ((rc = e.ensure(e.rasterImg, np * (shadow ? 1 : 4), err)) ||
-      (rc = e.ensure(e.rasterRows, rasterScratchBytes(n), err)))
+      (rc = e.ensure(e.rasterTall, rasterScratchBytes(n), err)))
     return rc;
-  if ((rc = rasterInto(e, cam, polys, root, tag, epoch, n, shadow, e.rasterImg.ptr, e.rasterRows.ptr, err))) return rc;
+  if ((rc = rasterInto(e, cam, polys, root, tag, epoch, n, shadow, e.rasterImg.ptr, e.rasterTall.ptr, err))) return rc;
   BTG_TRY(hipMemcpyAsync(hostOut, e.rasterImg.ptr, np * (shadow ? 1 : 4), hipMemcpyDeviceToHost, e.stream));
   BTG_TRY(hipStreamSynchronize(e.stream));
   return 0;

@@ -272,8 +272,8 @@ int btg_raster(btg_ctx* ctx, const btg_camera* cam, const btg_poly* polys, int64
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * polysDev: `count` btg_poly in device memory; idsDev (shadowPass = 0, W*H
  * int32) or maskDev (shadowPass = 1, W*H bytes) in device memory, written
- * with exactly btg_raster's result. The scan scratch is a static device array
- * sized for BTG_RASTER_NOALLOC_MAX_POLYS polygons (12 MiB), one per device,
+ * with exactly btg_raster's result. The scratch is a static device array
+ * sized for BTG_RASTER_NOALLOC_MAX_POLYS polygons (4 MiB), one per device,
  * held until the process ends; count above that maximum is BTG_ERR_LIMIT. All
  * calls on one device share that array: calls that overlap on one device race
  * (serialise them). Synchronous on the context's stream; device buffers the
