@@ -158,6 +158,16 @@ struct SoftJob {
   F3 lc, lU, lV;
 };
 
+// What a call reads back, in one block of device memory so that one copy to
+// pinned memory brings it: the pass state, the beams' and the primary rays'
+// counters, the phase clocks.
+// Before, a soft-shadow call read its counters twice through pageable memory,
+// waiting for the stream between its primary rays and its beams, and fetched its
+// images one by one: 0.60 ms for the room at 48 x 48, 0.41 ms now.
+constexpr size_t kStatBytes = size_t(kStatSlots) * kStatWords * 8;
+constexpr size_t kBackStats = (sizeof(WState) + 127) / 128 * 128, kBackRays = kBackStats + kStatBytes,
+                 kBackCycles = kBackRays + kStatBytes, kBackBytes = kBackCycles + 64;
+
 // An unoccluded soft-shadow piece waiting for its exact Lambert integral:
 // corners on its root's plane (lanes past n repeat the last), root, count.
 struct ShadeRec {
@@ -1982,6 +1992,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
   // the phases' LDS columns overlay each other: no lane holds a beam while its wave clips
   __shared__ uint32_t lds[kWaveWords * kBlock];
   __shared__ int shadeCounts[kBlock / kWave];
+  if (p.st->done) return;  // a launch past the pass's end
   const int n = int(min((unsigned long long)p.st->count[cur], p.capacity));
   const int nxt = cur ^ 1;
   const bool shade = isSoft(App) && p.exact;
@@ -3011,16 +3022,20 @@ class Engine {
   // scene storage
   void* sceneMem[7] = {};
   // engine buffers (grown on demand)
-  DevBuf tq0, tq1, sq, ws, roots, live, state, epoch, missFx, gFx, stats, st, out, outRoot, outTag, list, listCount;
-  DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, prim, retry, cycles, shq, jobs;
+  DevBuf tq0, tq1, sq, ws, roots, live, state, epoch, missFx, gFx, back, out, outRoot, outTag, list, listCount;
+  DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, img, prim, retry, shq, jobs;
   DevBuf valid, order, sorted;  // polygon lists on their way out: after retries, two orders, in canonical order
   // FP64 soft shadows: hit leaf reference per pixel; counters and cell lists;
   // the tracers' arrays; the jobs' double cameras; per-pixel fixed-point sums
   DevBuf pixRef, fpList, fpMem, camD, fpSum;
   DevBuf rasterImg, rasterTall;  // device rasterization: image; the list of the tall polygons
   void* noAllocScratch = nullptr;  // this device's static rasterization scratch (null: unavailable)
-  WState* hostState = nullptr;  // pinned
-  uint64_t phaseCycles[8] = {};
+  WState* hostState = nullptr;  // pinned: the last read-back of `back` (kBackBytes)
+  // Pinned memory on the way to and from the device, at most kStageMost bytes:
+  // copies of pageable memory wait for the stream and cost 30 us each.
+  void* stage = nullptr;
+  size_t stageBytes = 0;
+  const char* backAt(size_t off) const { return reinterpret_cast<const char*>(hostState) + off; }
   // per-launch timing (Options::profile): event pairs and the kernel kind
   std::vector<hipEvent_t> evPool;
   std::vector<int> evKind;
@@ -3052,6 +3067,24 @@ class Engine {
     evUsed = 0;
   }
 
+  // The stage with room for `bytes`, or null (more than kStageMost, or no pinned memory).
+  char* staging(size_t bytes) {
+    constexpr size_t kStageMost = size_t(4) << 20;
+    if (bytes > kStageMost) return nullptr;
+    if (stageBytes < bytes) {
+      if (stage) (void)hipHostFree(stage);
+      stage = nullptr;
+      stageBytes = 0;
+      const size_t want = bytes < (size_t(64) << 10) ? (size_t(64) << 10) : kStageMost;
+      if (hipHostMalloc(&stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        stage = nullptr;
+        return nullptr;
+      }
+      stageBytes = want;
+    }
+    return static_cast<char*>(stage);
+  }
   int ensure(DevBuf& b, size_t bytes, std::string& err) {
     if (b.bytes >= bytes && b.ptr) return 0;
     if (b.ptr) (void)hipFree(b.ptr);
@@ -3067,13 +3100,14 @@ class Engine {
     return 0;
   }
   ~Engine() {
-    DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &stats, &st, &out,
-                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterTall, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &prim, &valid, &order, &sorted, &retry, &cycles, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
+    DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &back, &out,
+                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterTall, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &img, &prim, &valid, &order, &sorted, &retry, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
     for (DevBuf* b : all)
       if (b->ptr) (void)hipFree(b->ptr);
     for (void* m : sceneMem)
       if (m) (void)hipFree(m);
     if (hostState) (void)hipHostFree(hostState);
+    if (stage) (void)hipHostFree(stage);
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : evPool) (void)hipEventDestroy(e);
@@ -3101,9 +3135,7 @@ int prepare(Engine& e, int app, int R, int budget, Params& p, std::string& err) 
       (rc = e.ensure(e.sq, cap * sizeof(Rec), err)) || (rc = e.ensure(e.roots, size_t(R) * sizeof(RootQ), err)) ||
       (rc = e.ensure(e.live, size_t(R) * 4, err)) || (rc = e.ensure(e.state, size_t(R) * 4, err)) ||
       (rc = e.ensure(e.epoch, size_t(R) * 4, err)) || (rc = e.ensure(e.missFx, size_t(R) * 8, err)) ||
-      (rc = e.ensure(e.gFx, size_t(R) * 8, err)) || (rc = e.ensure(e.stats, sizeof(uint64_t) * kStatSlots * kStatWords, err)) ||
-      (rc = e.ensure(e.st, sizeof(WState), err)) ||
-      (rc = e.ensure(e.cycles, 8 * sizeof(uint64_t), err)) ||
+      (rc = e.ensure(e.gFx, size_t(R) * 8, err)) || (rc = e.ensure(e.back, kBackBytes, err)) ||
       (rc = e.ensure(e.list, size_t(R) * 4, err)) || (rc = e.ensure(e.listCount, 4, err)))
     return rc;
   p = Params();
@@ -3126,9 +3158,10 @@ int prepare(Engine& e, int app, int R, int budget, Params& p, std::string& err) 
   p.pass = 0;
   p.missFx = static_cast<unsigned long long*>(e.missFx.ptr);
   p.gFx = static_cast<unsigned long long*>(e.gFx.ptr);
-  p.stats = static_cast<unsigned long long*>(e.stats.ptr);
-  p.cycles = static_cast<unsigned long long*>(e.cycles.ptr);
-  p.st = static_cast<WState*>(e.st.ptr);
+  char* const back = static_cast<char*>(e.back.ptr);
+  p.st = reinterpret_cast<WState*>(back);
+  p.stats = reinterpret_cast<unsigned long long*>(back + kBackStats);
+  p.cycles = reinterpret_cast<unsigned long long*>(back + kBackCycles);
   // Primary passes are chains of short rounds whose trace launches last as
   // long as their slowest lane: they yield after at most kPrimaryLeafCap
   // leaves (measured on the conference hall: 45 ms against 50 ms at 8).
@@ -3181,6 +3214,8 @@ constexpr int kFusedCheck = 4;               // fused rounds between state read-
 #endif
 constexpr int kReserveMin = 32, kReserveMax = BTG_RESERVE;  // at least what a root is admitted with (8 sign regions, fans of 3)
 
+int readBack(Engine& e, std::string& err);
+
 // Runs the rounds of one pass until the state reports done: groups of
 // roundsPerCheck rounds (admit, trace, shade, split each, or admit and the
 // fused kernel), then one state read-back. With Options::graphs each group is captured once into a HIP
@@ -3203,6 +3238,8 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
   // ever held). Roots
   // that find no room are abandoned and traced again with their budget reserved.
   p.reserve = p.rootList ? p.budget : std::min(std::max(p.budget, kReserveMin), kReserveMax);
+  // every root admitted at once (initKernel): the first round's launch is the only one
+  const bool atOnce = p.capacity / (unsigned long long)p.reserve >= (unsigned long long)p.R;
   bool admitting = true;
   auto group = [&](int first, int k, bool fused) {
     for (int i = 0; i < k; ++i) {
@@ -3212,6 +3249,7 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
         ls = e.beginLaunch(0);
         admitKernel<App><<<gA, kBlock, 0, e.stream>>>(p, cur);
         e.endLaunch(ls);
+        if (atOnce) admitting = false;
       }
       ls = e.beginLaunch(1);
       if (fused) {
@@ -3260,7 +3298,7 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
     }
     rounds += k;
     BTG_TRY(hipGetLastError());
-    BTG_TRY(hipMemcpyAsync(e.hostState, p.st, sizeof(WState), hipMemcpyDeviceToHost, e.stream));
+    if (int rc = readBack(e, err)) return rc;
     BTG_TRY(hipStreamSynchronize(e.stream));
     if (e.hostState->done) break;
     queued = (long long)e.hostState->count[rounds & 1] + e.hostState->admitCount;
@@ -3283,29 +3321,33 @@ int runPass(Engine& e, Params& p, RunInfo& info, std::string& err) {
   return runPassApp<kPoint>(e, p, info, err);
 }
 
-int readStats(Engine& e, uint64_t* dst, double* dropped, std::string& err) {
+// Sums the counter slots at `off` of the last read-back.
+void sumStats(const Engine& e, size_t off, uint64_t* dst, double* dropped) {
   static_assert(sNum < kStatWords, "a stat slot holds the counters and the dropped area");
-  std::vector<uint64_t> s(size_t(kStatSlots) * kStatWords);
-  BTG_TRY(hipMemcpyAsync(e.phaseCycles, e.cycles.ptr, sizeof(e.phaseCycles), hipMemcpyDeviceToHost, e.stream));
-  BTG_TRY(hipMemcpyAsync(s.data(), e.stats.ptr, s.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, e.stream));
-  BTG_TRY(hipStreamSynchronize(e.stream));
+  const char* slots = e.backAt(off);
   double d = 0;
   for (int k = 0; k < kStatSlots; ++k) {
-    const uint64_t* slot = s.data() + size_t(k) * kStatWords;
+    uint64_t slot[kStatWords];
+    std::memcpy(slot, slots + size_t(k) * sizeof(slot), sizeof(slot));
     for (int i = 0; i < sNum; ++i) dst[i] += slot[i];
     double x;
     std::memcpy(&x, slot + kStatWords - 1, sizeof(x));
     d += x;
   }
   if (dropped) *dropped += d;
-  return 0;
 }
 
 int zeroStats(Engine& e, std::string& err) {
-  zeroWords<<<kStatSlots * kStatWords / 256, 256, 0, e.stream>>>(static_cast<unsigned long long*>(e.stats.ptr),
-                                                               size_t(kStatSlots) * kStatWords);
-  zeroWords<<<1, 64, 0, e.stream>>>(static_cast<unsigned long long*>(e.cycles.ptr), 8);
+  constexpr size_t words = (kBackBytes - kBackStats) / 8;
+  zeroWords<<<(words + 255) / 256, 256, 0, e.stream>>>(
+      reinterpret_cast<unsigned long long*>(static_cast<char*>(e.back.ptr) + kBackStats), words);
   BTG_TRY(hipGetLastError());
+  return 0;
+}
+
+// Queues the read-back into the pinned copy.
+int readBack(Engine& e, std::string& err) {
+  BTG_TRY(hipMemcpyAsync(e.hostState, e.back.ptr, kBackBytes, hipMemcpyDeviceToHost, e.stream));
   return 0;
 }
 
@@ -3591,7 +3633,7 @@ Engine* engineCreate(const btg_scene_desc& d, float offset, float offsetGuard, s
   }
   (void)hipGetLastError();
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&e->hostState), sizeof(WState), hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc(reinterpret_cast<void**>(&e->hostState), kBackBytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     err = "stream / pinned allocation failed";
     delete e;
@@ -3770,12 +3812,14 @@ int engineSoftBatch(Engine* e, const SoftJobH* jobs, int n, bool exact, RunInfo&
   int rc = prepare(*e, guard ? kSoftG : kSoft, fp64Mode ? 0 : int(R), e->opt.budget, p, err);
   if (rc) return rc;
   const size_t np = size_t(npix);
-  if ((rc = e->ensure(e->pixTri, np * 4, err)) || (rc = e->ensure(e->pixX, np * 12, err)) ||
-      (rc = e->ensure(e->pixN, np * 12, err)) || (rc = e->ensure(e->vis, np * 4, err)) ||
-      (rc = e->ensure(e->E, np * 4, err)) || (rc = e->ensure(e->Eu, np * 4, err)) ||
-      (rc = e->ensure(e->jobs, jt.size() * sizeof(SoftJob), err)) ||
+  // the four output images one after the other, so that one copy takes them all
+  if ((rc = e->ensure(e->img, np * 16, err)) || (rc = e->ensure(e->pixX, np * 12, err)) ||
+      (rc = e->ensure(e->pixN, np * 12, err)) || (rc = e->ensure(e->jobs, jt.size() * sizeof(SoftJob), err)) ||
       (guard && (rc = e->ensure(e->pixXlo, np * 12, err))))
     return rc;
+  char* const img = static_cast<char*>(e->img.ptr);
+  // tables on their way to the device (at least as much as any call's images and results later)
+  char* const tables = e->staging(jt.size() * (sizeof(SoftJob) + 14 * sizeof(double)));
   if (guard) p.pixXlo = static_cast<const float*>(e->pixXlo.ptr);
   // FP64 mode: each job's camera in double (the caller's, or its floats widened)
   std::vector<double> camD;
@@ -3800,11 +3844,15 @@ int engineSoftBatch(Engine* e, const SoftJobH* jobs, int n, bool exact, RunInfo&
     if ((rc = e->ensure(e->pixRef, np * 4, err)) ||
         (rc = e->ensure(e->camD, camD.size() * sizeof(double), err)))
       return rc;
-    BTG_TRY(hipMemcpyAsync(e->camD.ptr, camD.data(), camD.size() * sizeof(double), hipMemcpyHostToDevice, e->stream));
+    const void* from = camD.data();
+    if (tables) from = std::memcpy(tables + jt.size() * sizeof(SoftJob), camD.data(), camD.size() * sizeof(double));
+    BTG_TRY(hipMemcpyAsync(e->camD.ptr, from, camD.size() * sizeof(double), hipMemcpyHostToDevice, e->stream));
     p.pixRef = static_cast<int*>(e->pixRef.ptr);
     p.jobCamD = static_cast<const double*>(e->camD.ptr);
   }
-  BTG_TRY(hipMemcpyAsync(e->jobs.ptr, jt.data(), jt.size() * sizeof(SoftJob), hipMemcpyHostToDevice, e->stream));
+  const void* from = jt.data();
+  if (tables) from = std::memcpy(tables, jt.data(), jt.size() * sizeof(SoftJob));
+  BTG_TRY(hipMemcpyAsync(e->jobs.ptr, from, jt.size() * sizeof(SoftJob), hipMemcpyHostToDevice, e->stream));
   p.jobs = static_cast<const SoftJob*>(e->jobs.ptr);
   p.numJobs = n;
   p.exact = exact ? 1 : 0;
@@ -3812,22 +3860,21 @@ int engineSoftBatch(Engine* e, const SoftJobH* jobs, int n, bool exact, RunInfo&
     if ((rc = e->ensure(e->shq, size_t(p.capacity) * sizeof(ShadeRec), err))) return rc;
     p.shq = static_cast<ShadeRec*>(e->shq.ptr);
   }
-  p.pixTri = static_cast<const int*>(e->pixTri.ptr);
+  p.pixTri = reinterpret_cast<const int*>(img);
   p.pixX = static_cast<const float*>(e->pixX.ptr);
   p.pixN = static_cast<const float*>(e->pixN.ptr);
-  p.vis = static_cast<float*>(e->vis.ptr);
-  p.E = static_cast<float*>(e->E.ptr);
-  p.Eu = static_cast<float*>(e->Eu.ptr);
+  p.vis = reinterpret_cast<float*>(img + np * 4);
+  p.E = reinterpret_cast<float*>(img + np * 8);
+  p.Eu = reinterpret_cast<float*>(img + np * 12);
   if ((rc = zeroStats(*e, err))) return rc;
   BTG_TRY(hipEventRecord(e->ev[0], e->stream));
   const int lp = e->beginLaunch(3);
-  primaryRayKernel<<<unsigned(tiles), kRayBlock, 0, e->stream>>>(p);
+  Params rays = p;  // the primary pass's counters are reported separately
+  rays.stats = reinterpret_cast<unsigned long long*>(static_cast<char*>(e->back.ptr) + kBackRays);
+  primaryRayKernel<<<unsigned(tiles), kRayBlock, 0, e->stream>>>(rays);
   e->endLaunch(lp);
   BTG_TRY(hipGetLastError());
   BTG_TRY(hipEventRecord(e->ev[1], e->stream));
-  // the primary pass's counters are reported separately
-  if ((rc = readStats(*e, info.rayStats, nullptr, err))) return rc;
-  if ((rc = zeroStats(*e, err))) return rc;
   BTG_TRY(hipEventRecord(e->ev[2], e->stream));
   auto fin = [&](Params& q) -> int {
     finalizeSoftKernel<<<(q.R + 255) / 256, 256, 0, e->stream>>>(q);
@@ -3835,30 +3882,42 @@ int engineSoftBatch(Engine* e, const SoftJobH* jobs, int n, bool exact, RunInfo&
     return 0;
   };
   if (fp64Mode) {
-    if ((rc = softFp64(*e, p, np, err))) return rc;
+    if ((rc = softFp64(*e, p, np, err)) || (rc = readBack(*e, err))) return rc;
   } else if ((rc = runAll(*e, p, e->opt.budget, info, fin, err))) {
     return rc;
   }
   BTG_TRY(hipEventRecord(e->ev[3], e->stream));
-  BTG_TRY(hipEventSynchronize(e->ev[3]));
+  bool wanted = false;
+  for (int j = 0; j < n; ++j) wanted = wanted || jobs[j].tri || jobs[j].vis || jobs[j].E || jobs[j].Eu;
+  // small images through the stage in one copy, larger ones straight to their arrays
+  char* const small = wanted ? e->staging(np * 16) : nullptr;
+  if (small) {
+    BTG_TRY(hipMemcpyAsync(small, img, np * 16, hipMemcpyDeviceToHost, e->stream));
+    BTG_TRY(hipStreamSynchronize(e->stream));
+  }
+  for (int j = 0; j < n; ++j) {
+    const SoftJobH& h = jobs[j];
+    const SoftJob& J = jt[size_t(j)];
+    const size_t off = size_t(J.pixBase) * 4, bytes = size_t(J.W) * size_t(J.H) * 4;
+    void* const to[4] = {h.tri, h.vis, h.E, h.Eu};
+    for (size_t k = 0; k < 4; ++k) {
+      if (!to[k]) continue;
+      if (small)
+        std::memcpy(to[k], small + k * np * 4 + off, bytes);
+      else
+        BTG_TRY(hipMemcpyAsync(to[k], img + k * np * 4 + off, bytes, hipMemcpyDeviceToHost, e->stream));
+    }
+  }
+  BTG_TRY(hipStreamSynchronize(e->stream));
   float ms0 = 0, ms1 = 0;
   BTG_TRY(hipEventElapsedTime(&ms0, e->ev[0], e->ev[1]));
   BTG_TRY(hipEventElapsedTime(&ms1, e->ev[2], e->ev[3]));
   info.primaryMs += ms0;
   info.traceMs += ms1;
-  if ((rc = readStats(*e, info.stats, &info.dropped, err))) return rc;
-  for (int k = 0; k < 8; ++k) info.phaseCycles[k] = e->phaseCycles[k];
+  sumStats(*e, kBackRays, info.rayStats, nullptr);
+  sumStats(*e, kBackStats, info.stats, &info.dropped);
+  std::memcpy(info.phaseCycles, e->backAt(kBackCycles), sizeof(info.phaseCycles));
   e->collectLaunches(info);
-  for (int j = 0; j < n; ++j) {
-    const SoftJobH& h = jobs[j];
-    const SoftJob& J = jt[size_t(j)];
-    const size_t off = size_t(J.pixBase), cnt = size_t(J.W) * size_t(J.H);
-    if (h.tri) BTG_TRY(hipMemcpyAsync(h.tri, static_cast<int*>(e->pixTri.ptr) + off, cnt * 4, hipMemcpyDeviceToHost, e->stream));
-    if (h.vis) BTG_TRY(hipMemcpyAsync(h.vis, static_cast<float*>(e->vis.ptr) + off, cnt * 4, hipMemcpyDeviceToHost, e->stream));
-    if (h.E) BTG_TRY(hipMemcpyAsync(h.E, static_cast<float*>(e->E.ptr) + off, cnt * 4, hipMemcpyDeviceToHost, e->stream));
-    if (h.Eu) BTG_TRY(hipMemcpyAsync(h.Eu, static_cast<float*>(e->Eu.ptr) + off, cnt * 4, hipMemcpyDeviceToHost, e->stream));
-  }
-  BTG_TRY(hipStreamSynchronize(e->stream));
   // triangle ids back to each job's scene numbering
   for (int j = 0; j < n; ++j) {
     const SoftJobH& h = jobs[j];
@@ -3882,7 +3941,7 @@ Engine* engineShare(Engine* base, std::string& err) {
   e->cus = base->cus;
   e->opt = base->opt;
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&e->hostState), sizeof(WState), hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc(reinterpret_cast<void**>(&e->hostState), kBackBytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     err = "stream / pinned allocation failed";
     delete e;
@@ -4355,18 +4414,18 @@ int runPolys(Engine& e, int app, int R, int budget, size_t outCap, const HostCam
     auto fin = [&](Params&) -> int { return 0; };
     if ((rc = runAll(e, p, budget, ri, fin, err))) return rc;
     BTG_TRY(hipEventRecord(e.ev[1], e.stream));
-    BTG_TRY(hipEventSynchronize(e.ev[1]));
     if (e.hostState->outCount > p.outCap) {
       outCap = size_t(e.hostState->outCount) + size_t(e.hostState->outCount) / 4;
       e.evUsed = 0;
       continue;
     }
+    sumStats(e, kBackStats, ri.stats, &ri.dropped);
+    if (download && (rc = takePolys(e, ri.retries > 0, canonical, polys, err))) return rc;
+    BTG_TRY(hipEventSynchronize(e.ev[1]));
     float ms = 0;
     BTG_TRY(hipEventElapsedTime(&ms, e.ev[0], e.ev[1]));
     ri.traceMs = ms;
-    if ((rc = readStats(e, ri.stats, &ri.dropped, err))) return rc;
     e.collectLaunches(ri);
-    if (download && (rc = takePolys(e, ri.retries > 0, canonical, polys, err))) return rc;
     info = ri;
     return 0;
   }
@@ -4694,8 +4753,11 @@ int rasterDevice(Engine& e, const HostCam& cam, const OutPoly* polys, const int*
       (rc = e.ensure(e.rasterTall, rasterScratchBytes(n), err)))
     return rc;
   if ((rc = rasterInto(e, cam, polys, root, tag, epoch, n, shadow, e.rasterImg.ptr, e.rasterTall.ptr, err))) return rc;
-  BTG_TRY(hipMemcpyAsync(hostOut, e.rasterImg.ptr, np * (shadow ? 1 : 4), hipMemcpyDeviceToHost, e.stream));
+  const size_t bytes = np * (shadow ? 1 : 4);
+  char* const small = e.staging(bytes);
+  BTG_TRY(hipMemcpyAsync(small ? small : hostOut, e.rasterImg.ptr, bytes, hipMemcpyDeviceToHost, e.stream));
   BTG_TRY(hipStreamSynchronize(e.stream));
+  if (small) std::memcpy(hostOut, small, bytes);
   return 0;
 }
 
