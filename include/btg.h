@@ -75,8 +75,11 @@ const char* btg_last_error(const btg_ctx* ctx);
 /* Engine knobs (cuda/gpu_render.h:48-58): budget = live sub-beams per soft /
  * point root (wfBudget, 128), primaryBudget = per primary tile (4096),
  * capacity = sub-beam records per queue (wfCapacity, 1 << 23),
- * roundsPerCheck = rounds launched between completion checks.
- * Roots over budget are not sent to the CPU: they are traced again on the GPU
+ * roundsPerCheck = rounds launched between completion checks, at most: rounds
+ * whose queue does not fill the device are checked every four at the latest.
+ * A first run reserves 32 to 128 records of the capacity per root (at most the
+ * budget above 32); a root that finds no room is traced again with its budget
+ * reserved. Roots over budget are not sent to the CPU: they are traced again on the GPU
  * with a larger budget. */
 typedef struct {
   int budget;
@@ -85,7 +88,8 @@ typedef struct {
   int roundsPerCheck;
   int profileKernels; /* 1: time every launch with HIP events (btg_run_info.kernelSeconds) */
   int leafCap;        /* leaves a sub-beam visits per trace launch before it yields to the next round (0: no cap);
-                         primary-visibility passes use at most 4 (latency-bound chains of short rounds) */
+                         primary-visibility passes use at most 4. Rounds whose queue does not fill the device
+                         run as one launch (trace and clips together), which this does not bound */
   int precision;      /* soft shadows: 0 = the reference's float build, bit for bit (default); 1 = FP64-guarded:
                          the receiver point is the primary ray's hit computed in double, the beam apex sits at
                          the double build's offset (1e-9 x scene extent) from it, formed in double and carried as
@@ -97,8 +101,8 @@ typedef struct {
                          job's double camera (btg_soft_job.camD) every visible fraction is bt_render_d's to
                          ~1e-10. Tens of times slower than 0; a server on such a context serves its soft
                          requests in FP64 batches (see btg_server_create). */
-  int useGraphs;      /* 1 (default): each group of roundsPerCheck rounds is captured once per pass into a HIP graph
-                         and replayed (no counterpart in the reference, which launches every kernel from the host,
+  int useGraphs;      /* 1 (default): each full group of roundsPerCheck rounds of separate launches is captured once
+                         per pass into a HIP graph and replayed (no counterpart in the reference, which launches every kernel from the host,
                          cuda/wavefront.cu:641-676); 0: plain launches. Results are the same either way.
                          profileKernels = 1 launches directly (it times every launch with HIP events).
                          While a pass captures (microseconds per group), operations that other threads of
@@ -158,7 +162,8 @@ typedef struct {
   btg_trace_stats stats;  /* beam counters (engine-independent) */
   btg_trace_stats rayStats;
   /* with profileKernels: summed launch durations and launch counts per kernel
-   * (0 admit, 1 trace, 2 split, 3 primary rays, 4 other) */
+   * (0 admit, 1 trace, 2 split, 3 primary rays, 4 other); a round of one launch
+   * counts as trace */
   double kernelSeconds[5];
   int kernelLaunches[5];
   /* builds with -DBTG_PHASE_CYCLES: trace-loop clocks spent refilling,
