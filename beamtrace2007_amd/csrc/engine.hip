@@ -2837,6 +2837,12 @@ __global__ void zeroWords(unsigned long long* w, size_t n) {
 // threads). A finished cell adds its results to the pixel's fixed-point sums;
 // a cell over the work cap or the pools goes to `out` for the next level (on
 // level 2, which has no cap, it counts in *failed, as does a full `out`).
+// Fewer tasks than lanes are spread over all waves, as many lanes of each
+// working as it takes: a wave's lanes do different things one after the other,
+// so that a task among 8 takes a fraction of its time among 64: two images of
+// sides 48 to 64 of the conference hall 42.8 -> 22.8 ms, of the atrium 28.9 -> 11.4
+// ms, one of 96 x 90 of the building 57.7 -> 44.0 ms; batches of more roots than
+// lanes the same.
 template <int Pn, int Kn, int Level>
 __global__ void __launch_bounds__(64, kFp64Waves)
     fp64CellKernel(Params p, int numPix, const long long* in, const int* inCount, int inCap, int* next, uint64_t* mem,
@@ -2847,7 +2853,8 @@ __global__ void __launch_bounds__(64, kFp64Waves)
   tr.cnt.zero();
   tr.m = fp64::WordMem{mem + size_t(blockIdx.x) * size_t(TR::kWords) * 64, 64, int(threadIdx.x)};
   const int tasks = Level == 0 ? numPix : 16 * min(*inCount, inCap);
-  for (;;) {
+  const int lanes = (tasks + int(gridDim.x) - 1) / int(gridDim.x);
+  for (; int(threadIdx.x) < lanes;) {
     const int t = atomicAdd(next, 1);
     if (t >= tasks) break;
     int pix = t, cx = 0, cy = 0;
@@ -3738,7 +3745,7 @@ int softFp64(Engine& e, Params& p, size_t np, std::string& err) {
   constexpr size_t kBlock0 = size_t(T0::kWords) * 64 * 8, kBlock1 = size_t(T1::kWords) * 64 * 8,
                    kBlock2 = size_t(T2::kWords) * 64 * 8;
   const size_t cus = size_t(std::max(e.cus, 1)), maxBlocks = cus * 4 * kFp64Waves;
-  const size_t blocks0 = std::min((np + 63) / 64, maxBlocks);
+  const size_t blocks0 = std::min(np, maxBlocks);  // (its memory: less than blocks2 takes)
   const size_t blocks1 = std::min((16 * np + 63) / 64, maxBlocks);
   // every level fills the device's SIMDs (level 2 on one wave per CU took 1.35 times as long on the plant)
   const size_t blocks2 = std::min((256 * np + 63) / 64, maxBlocks);
