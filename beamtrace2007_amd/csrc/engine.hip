@@ -2813,9 +2813,13 @@ constexpr int kFp64Waves = BTG_FP64_WAVES;
 // six conference jobs of sides 64 to 96 319 / - / 214 / 214 / 243 / 303, the plant
 // at 160 x 160 828 / - / 648 / 628 / 590 / 562, the room at 48 to 64 3.3 / - / 3.3 /
 // 3.3 / 4.6 / 6.3: below 384 the cells' repeated set-up costs the cheap scenes more
-// than the shorter tail gives them.
+// than the shorter tail gives them. With small levels spread over all waves, 384 /
+// 512 / 2048 (the last without the spread): eight room images of 96 to 128 8.6 /
+// 6.7 / 6.9, of 48 to 88 6.9 / 5.9 / 6.0, eight conference images of 96 to 128 378 /
+// 353 / 416, of the building at 48 to 88 74 / 85 / 182, the atrium 407 / 422 / 636:
+// 512 costs no scene of cheap roots more than the tail saves it.
 #ifndef BTG_FP64_WORK_CAP
-#define BTG_FP64_WORK_CAP 384
+#define BTG_FP64_WORK_CAP 512
 #endif
 constexpr uint32_t kFp64WorkCap = BTG_FP64_WORK_CAP;
 // Beams and work items of a level-1 cell's pools (build knob BTG_FP64_POOL1).
