@@ -39,6 +39,7 @@
 
 #include "engine.h"
 #include "kd_pred.h"
+#include "poly_order.h"
 
 // Scratch of the allocation-free rasterization (btg_raster_device_noalloc): a
 // count and a number (4 B) for each of kNoAllocMaxPolys polygons, 4 MiB. Every
@@ -4293,19 +4294,6 @@ int openCollect(OpenPass* op, std::vector<int>& completed, std::vector<int>& kil
 namespace {
 
 // ---------------------------------------------------------- canonical order
-// polyLess of the reference's canonical list: triangle, corner count, corners, area.
-__device__ __forceinline__ bool polyLess(const OutPoly& a, const OutPoly& b) {
-  if (a.tri != b.tri) return a.tri < b.tri;
-  if (a.n != b.n) return a.n < b.n;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= a.n) break;
-    if (a.x[k] != b.x[k]) return a.x[k] < b.x[k];
-    if (a.y[k] != b.y[k]) return a.y[k] < b.y[k];
-  }
-  return a.area < b.area;
-}
-
 // The sort works on polygon numbers: blocks of kSortBlock put in order by
 // counting, then runs merged pairwise, every element finding its place by a
 // binary search of its sibling run. Most comparisons end at the triangle. Both
@@ -4324,10 +4312,7 @@ __global__ void __launch_bounds__(kSortBlock) sortBlocks(const OutPoly* polys, i
   for (int j = 0; j < m; ++j) {
     const int t = tris[j];
     bool before = t < own.tri;
-    if (t == own.tri && base + j != i) {
-      const OutPoly other = polys[base + j];
-      before = polyLess(other, own) || (base + j < i && !polyLess(own, other));
-    }
+    if (t == own.tri && base + j != i) before = goesBefore(polys[base + j], base + j, own, i);
     rank += before;
   }
   order[base + rank] = i;
@@ -4342,16 +4327,8 @@ __global__ void __launch_bounds__(256) mergeRuns(const OutPoly* polys, const int
   const OutPoly own = polys[k];
   int lo = 0;
   if (sib < n) {
-    int hi = int(min(int64_t(run), int64_t(n) - sib));
-    const bool second = mine & 1;  // elements of the first run precede their equals
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      const OutPoly other = polys[in[sib + mid]];
-      if (second ? !polyLess(own, other) : polyLess(other, own))
-        lo = mid + 1;
-      else
-        hi = mid;
-    }
+    const int count = int(min(int64_t(run), int64_t(n) - sib));
+    lo = mergeBefore(own, (mine & 1) != 0, count, [&](int m) { return polys[in[sib + m]]; });
   }
   out[(mine & ~1) * int64_t(run) + (i - begin) + lo] = k;
 }
