@@ -3501,12 +3501,15 @@ SceneRec makeSceneRec(const btg_scene_desc& d, float offset, float offsetGuard) 
 }
 
 // Each leaf's ancestors, root first, at the base its split field holds: the
-// leaf's depth entries of (node, data word).
+// leaf's depth entries of (node, data word). Nodes that no descent reaches have
+// none (kNoAncestors): a scene's checks ask nothing of their parent links but
+// their range, so they may run in circles.
+constexpr uint32_t kNoAncestors = 0xffffffffu;
 __global__ void fillAncestors(DevScene sv, uint32_t nodes, uint2* anc) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nodes) return;
   const KdNodeD leaf = sv.nodes[i];
-  if ((leaf.data & 3u) != 3u) return;
+  if ((leaf.data & 3u) != 3u || __float_as_uint(leaf.split) == kNoAncestors) return;
   uint32_t depth = 0;
   for (uint32_t k = i, up; (up = sv.parent[k]) != k; k = up) ++depth;
   uint2* const list = anc + __float_as_uint(leaf.split);
@@ -3541,9 +3544,8 @@ int rebuildArena(Engine& e, std::string& err) {
   std::vector<uint32_t> par;
   std::vector<LeafTri> lt;
   std::vector<int32_t> rt;
-  std::vector<uint32_t> depths;  // of the arena's nodes (a parent is numbered before its children)
+  std::vector<int32_t> depth;  // of a scene's nodes (children follow their parent); -1: not reached
   uint64_t ancEntries = 0;
-  depths.reserve(nodes);
   nv.reserve(size_t(tris) * 2);
   kn.reserve(nodes);
   bx.reserve(nodes);
@@ -3554,17 +3556,19 @@ int rebuildArena(Engine& e, std::string& err) {
     if (!sr.live) continue;
     const uint64_t anc0 = ancEntries;
     nv.insert(nv.end(), sr.triNV.begin(), sr.triNV.end());
+    depth.assign(sr.nodes.size(), -1);
+    depth[0] = 0;
     for (size_t i = 0; i < sr.nodes.size(); ++i) {
       KdNodeD n = sr.nodes[i];
-      const uint32_t depth = i == 0 ? 0u : depths[sr.nodeBase + sr.parent[i]] + 1u;
-      depths.push_back(depth);
       if ((n.data & 3u) != 3u) {
+        if (depth[i] >= 0) depth[i + 1] = depth[n.data >> 2] = depth[i] + 1;
         n.data = (n.data & 3u) | (((n.data >> 2) + sr.nodeBase) << 2);
       } else {
         n.offset += sr.refBase;
-        const uint32_t base = uint32_t(ancEntries);  // a leaf's split field is unused: its ancestors' first entry
+        // a leaf's split field is unused: its ancestors' first entry
+        const uint32_t base = depth[i] >= 0 ? uint32_t(ancEntries) : kNoAncestors;
         std::memcpy(&n.split, &base, sizeof(base));
-        ancEntries += depth;
+        if (depth[i] > 0) ancEntries += uint32_t(depth[i]);
       }
       kn.push_back(n);
       par.push_back(i == 0 ? sr.nodeBase : sr.parent[i] + sr.nodeBase);
@@ -3592,10 +3596,10 @@ int rebuildArena(Engine& e, std::string& err) {
   if (!rc) rc = upload(e, 5, rt.data(), rt.size(), sv.refTri, err);
   if (rc) return rc;
   // The ancestor lists are filled on the device from the parent links. Without
-  // room for them (or with more entries than 32 bits number) climbs follow
+  // room for them (or with more entries than their numbers allow) climbs follow
   // the parent links instead.
   sv.anc = nullptr;
-  if (ancEntries > 0 && ancEntries < (1ull << 32)) {
+  if (ancEntries > 0 && ancEntries < kNoAncestors) {
     void* d = nullptr;
     if (hipMalloc(&d, size_t(ancEntries) * sizeof(uint2)) == hipSuccess) {
       e.sceneMem[6] = d;
