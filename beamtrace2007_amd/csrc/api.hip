@@ -627,7 +627,7 @@ struct btg_server {
   std::unordered_map<int, SrvReq*> slots[2];  // pass slot -> request
   int active = 0;                             // the pass that takes new requests
   btg::Engine* pointEngine = nullptr;
-  btg::Engine* fallback = nullptr;            // re-runs a request whose roots went over budget
+  btg::Engine* fallback = nullptr;            // re-runs a request some of whose roots were abandoned
   std::mutex m;
   std::condition_variable cvSoft, cvPoint, cvDone;
   std::deque<SrvReq*> softQ, pointQ;
@@ -749,7 +749,7 @@ void softLoop(btg_server* s) {
         }
         if (!r) continue;  // a slot the server never filled: nothing waits on it
         int rc = BTG_OK;
-        if (killed[i] > 0) {  // over budget: trace the request again alone, with GPU retries
+        if (killed[i] > 0) {  // over budget or without room: trace the request again alone, with GPU retries
           btg::SoftJobH h = jobOf(r->req);
           btg::RunInfo ri;
           rc = btg::engineSoftBatch(s->fallback, &h, 1, true, ri, err);

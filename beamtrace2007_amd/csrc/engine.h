@@ -206,7 +206,7 @@ int openTryAdd(OpenPass* op, const SoftJobH& job, int* slot, std::string& err);
 // Launches `rounds` rounds and an asynchronous read-back of the job counters.
 int openStep(OpenPass* op, int rounds, std::string& err);
 // Waits for the last step; finalizes and downloads the jobs that completed
-// since (their slots, and per slot the roots that went over budget).
+// since (their slots, and per slot the roots that were abandoned).
 int openCollect(OpenPass* op, std::vector<int>& completed, std::vector<int>& killed, std::string& err);
 int openJobs(const OpenPass* op);
 bool openIdle(const OpenPass* op);

@@ -70,7 +70,9 @@ constexpr int kMbox = 8;            // mailbox entries per lane (a power of two)
 // double build's apex offset, the apex held as a float pair).
 enum App { kSoft = 0, kPrimary = 1, kPoint = 2, kSoftG = 3 };
 constexpr bool isSoft(int app) { return app == kSoft || app == kSoftG; }
-enum RootState { kTraced = 0, kKilled = 1, kNoBeam = 2 };
+// kKilled: abandoned over its budget; kNoRoom: abandoned because a queue was full.
+enum RootState { kTraced = 0, kKilled = 1, kNoBeam = 2, kNoRoom = 3 };
+constexpr int kAbandonedBit = 1;  // of both states of an abandoned root, and of no other
 enum { kKeep = 0, kAllIn = 1, kClip = 2 };
 enum { kFinished = 0, kSplit = 1, kContinue = 2 };
 enum { kDescend = 0, kTest = 1, kClimb = 2 };
@@ -1031,8 +1033,14 @@ __device__ __forceinline__ void rootDone(const Params& p, int root) {
 __device__ __forceinline__ void liveSub(const Params& p, int root, int n) {
   if (atomicSub(&p.live[root], n) == n) rootDone(p, root);
 }
+__device__ __forceinline__ bool abandoned(int state) { return (state & kAbandonedBit) != 0; }
+// A root over its budget (also if it found no room before: it needs the larger
+// budget), and one that found no room.
 __device__ __forceinline__ void killRoot(const Params& p, int root) {
-  if (atomicExch(&p.state[root], int(kKilled)) != int(kKilled)) atomicAdd(&p.st->killed, 1);
+  if (!abandoned(atomicExch(&p.state[root], int(kKilled)))) atomicAdd(&p.st->killed, 1);
+}
+__device__ __forceinline__ void noRoomFor(const Params& p, int root) {
+  if (atomicCAS(&p.state[root], int(kTraced), int(kNoRoom)) == int(kTraced)) atomicAdd(&p.st->killed, 1);
 }
 
 // Where a wave of the fused kernel puts the pieces that wait for their Lambert
@@ -1070,7 +1078,7 @@ __device__ __forceinline__ void emitOutput(const Params& p, const Ctx& c, const 
         if ((unsigned long long)k < p.capacity)
           p.shq[k] = sr;
         else
-          killRoot(p, root);
+          noRoomFor(p, root);
       }
     }
     return;
@@ -1102,7 +1110,7 @@ __device__ __forceinline__ void toQueue(const Params& p, int q, int slot, const 
   if ((unsigned long long)slot < p.capacity) {
     p.tq[q][slot] = r;
   } else {
-    killRoot(p, r.root);
+    noRoomFor(p, r.root);
     liveSub(p, r.root, 1);
   }
 }
@@ -1111,7 +1119,7 @@ __device__ __forceinline__ void toQueue(const Params& p, int q, int slot, const 
 __device__ __forceinline__ Rec* roomAt(const Params& p, int q, int slot, int slots, int root) {
   if ((unsigned long long)(slot + slots) <= p.capacity) return p.tq[q] + slot;
   if (slots > 0) {
-    killRoot(p, root);
+    noRoomFor(p, root);
     int lost = slots;
     for (int k = 0; k < slots && (unsigned long long)(slot + k) < p.capacity; ++k, --lost) {
       p.tq[q][slot + k].n = 0;
@@ -1588,7 +1596,7 @@ __device__ __forceinline__ int coopTest(const Params& p, const Ctx& c, Rec& r, W
 template <int App>
 __device__ __forceinline__ bool loadBeam(const Params& p, Ctx& c, const Rec& r, Work& w, Stepper& ss, float* bounds,
                                          int32_t* mboxLds) {
-  if (r.n == 0 || p.state[r.root] == kKilled) {
+  if (r.n == 0 || abandoned(p.state[r.root])) {
     liveSub(p, r.root, 1);
     return false;
   }
@@ -1786,7 +1794,7 @@ __device__ __forceinline__ void clipChunk(const Params& p, bool valid, const Rec
   int staged = -1;  // pieces kept in LDS by the counting pass (-1: clip again)
   int tri = -1;
   if (valid) {
-    if (p.state[r.root] == kKilled) {
+    if (abandoned(p.state[r.root])) {
       liveSub(p, r.root, 1);
     } else {
       c = modeCtx<App>(p.roots[r.root]);
@@ -2550,7 +2558,8 @@ __device__ void admitRoot(const Params& p, int k, int cur, Cnt& cnt) {
   AdmitOut ao{0, true, node0, bounds};
   admitPoly<App>(p, c, poly, k, cur, ao, cnt);
   p.live[k] = ao.pushed;
-  if (!ao.ok || ao.pushed > p.budget) killRoot(p, k);
+  if (!ao.ok) noRoomFor(p, k);
+  if (ao.pushed > p.budget) killRoot(p, k);
   if (ao.pushed == 0) rootDone(p, k);
 }
 
@@ -2582,7 +2591,7 @@ __device__ __forceinline__ int finalizeRoot(const Params& p, int k) {
   int pix;
   if (!softPixel(p.jobs[jobOfRoot(p, k)], k, pix)) return kNoBeam;
   const int s = p.state[k];
-  if (s != kTraced) return s;  // no beam (written at admission) or killed (traced again)
+  if (s != kTraced) return s;  // no beam (written at admission) or abandoned (traced again)
   const RootQ& R = p.roots[k];
   const double miss = double(p.missFx[k]) * pow2(R.unitExp);
   const float V0 = float(miss) / R.lightArea;
@@ -2600,23 +2609,23 @@ __global__ void finalizeSoftKernel(Params p) {
 }
 
 // finalizeSoftKernel over the roots [begin, begin + count) of one job of an
-// open pass, plus the number of them that were abandoned (over budget).
+// open pass, plus the number of them that were abandoned.
 __global__ void finalizeRangeKernel(Params p, int begin, int count, int* killed) {
   const int i = int(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= count) return;
-  if (finalizeRoot(p, begin + i) == kKilled) atomicAdd(killed, 1);
+  if (abandoned(finalizeRoot(p, begin + i))) atomicAdd(killed, 1);
 }
 
 __global__ void clearInt(int* x) {
   if (threadIdx.x == 0) *x = 0;
 }
 
-// Killed roots, compacted for a retry pass.
-__global__ void collectKilled(Params p, int* list, int* count) {
-  const int i = int(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= p.R) return;
-  const int k = p.rootList ? p.rootList[i] : i;
-  if (p.state[k] == kKilled) list[atomicAdd(count, 1)] = k;
+// Abandoned roots, compacted for a retry pass: all of them, or those that found no room.
+__global__ void collectAbandoned(Params p, bool all, int* list, int* count) {
+  const int k = int(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k >= p.R) return;
+  const int s = p.state[k];
+  if (all ? abandoned(s) : s == kNoRoom) list[atomicAdd(count, 1)] = k;
 }
 
 // ------------------------------------------------------------ primary rays
@@ -3056,7 +3065,7 @@ class Engine {
   void* sceneMem[7] = {};
   // engine buffers (grown on demand)
   DevBuf tq0, tq1, sq, ws, roots, live, state, epoch, missFx, gFx, back, out, outRoot, outTag, list, listCount;
-  DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, img, prim, retry, shq, jobs;
+  DevBuf pixTri, pixX, pixXlo, pixN, vis, E, Eu, img, prim, shq, jobs;
   DevBuf valid, order, sorted;  // polygon lists on their way out: after retries, two orders, in canonical order
   // FP64 soft shadows: hit leaf reference per pixel; counters and cell lists;
   // the tracers' arrays; the jobs' double cameras; per-pixel fixed-point sums
@@ -3134,7 +3143,7 @@ class Engine {
   }
   ~Engine() {
     DevBuf* all[] = {&tq0, &tq1, &sq, &ws, &roots, &live, &state, &epoch, &missFx, &gFx, &back, &out,
-                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterTall, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &img, &prim, &valid, &order, &sorted, &retry, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
+                     &outRoot, &outTag, &list, &listCount, &rasterImg, &rasterTall, &pixTri, &pixX, &pixXlo, &pixN, &vis, &E, &Eu, &img, &prim, &valid, &order, &sorted, &shq, &jobs, &pixRef, &fpList, &fpMem, &camD, &fpSum};
     for (DevBuf* b : all)
       if (b->ptr) (void)hipFree(b->ptr);
     for (void* m : sceneMem)
@@ -3386,8 +3395,24 @@ int readBack(Engine& e, std::string& err) {
   return 0;
 }
 
-// The main pass plus GPU retry passes for roots over budget. `finalize`
-// runs after each pass over that pass's roots.
+// Collects the roots of pass p still abandoned into e.list (all of them, or
+// those that found no room).
+int collectRoots(Engine& e, const Params& p, bool all, int& n, std::string& err) {
+  clearInt<<<1, 64, 0, e.stream>>>(static_cast<int*>(e.listCount.ptr));
+  collectAbandoned<<<(p.R + 255) / 256, 256, 0, e.stream>>>(p, all, static_cast<int*>(e.list.ptr),
+                                                            static_cast<int*>(e.listCount.ptr));
+  BTG_TRY(hipGetLastError());
+  BTG_TRY(hipMemcpyAsync(&n, e.listCount.ptr, 4, hipMemcpyDeviceToHost, e.stream));
+  BTG_TRY(hipStreamSynchronize(e.stream));
+  return 0;
+}
+
+// The main pass plus GPU retry passes for the roots it abandoned. Roots that
+// found no room, in a first run that reserved less than their budget, are traced
+// again with that budget reserved: it then suffices, unless they go over it,
+// and as many run at once as the reference's rule admits. Roots over
+// their budget are traced again with 32 times as much, all that is left
+// together. `finalize` runs after each pass over that pass's roots.
 template <class Finalize>
 int runAll(Engine& e, Params& p, int baseBudget, RunInfo& info, Finalize finalize, std::string& err) {
   int rc = runPass(e, p, info, err);
@@ -3395,38 +3420,31 @@ int runAll(Engine& e, Params& p, int baseBudget, RunInfo& info, Finalize finaliz
   if ((rc = finalize(p))) return rc;
   info.killed = e.hostState->killed;
   int budget = baseBudget;
-  while (e.hostState->killed > 0) {
-    // Collect the killed roots and trace them again with a larger budget.
-    clearInt<<<1, 64, 0, e.stream>>>(static_cast<int*>(e.listCount.ptr));
-    collectKilled<<<(p.R + 255) / 256, 256, 0, e.stream>>>(p, static_cast<int*>(e.list.ptr),
-                                                             static_cast<int*>(e.listCount.ptr));
-    BTG_TRY(hipGetLastError());
+  bool whole = p.reserve >= budget;  // the last run had whole budgets reserved
+  for (int left = e.hostState->killed; left > 0; left += e.hostState->killed) {
     int nk = 0;
-    BTG_TRY(hipMemcpyAsync(&nk, e.listCount.ptr, 4, hipMemcpyDeviceToHost, e.stream));
-    BTG_TRY(hipStreamSynchronize(e.stream));
-    if (nk == 0) break;
-    // (after a first run that reserved less than the budget, the budget itself is still to be tried)
-    if ((unsigned long long)budget >= p.capacity && p.reserve >= budget) {
-      err = "a root needs more sub-beams than the queue capacity (" + std::to_string(p.capacity) + ")";
-      return BTG_ERR_LIMIT_CODE;
+    if (!whole && (rc = collectRoots(e, p, false, nk, err))) return rc;
+    if (nk > 0) {
+      budget = int(std::min<unsigned long long>((unsigned long long)budget, p.capacity));
+    } else {
+      if ((rc = collectRoots(e, p, true, nk, err))) return rc;
+      if (nk == 0) break;
+      if ((unsigned long long)budget >= p.capacity && whole) {
+        err = "a root needs more sub-beams than the queue capacity (" + std::to_string(p.capacity) + ")";
+        return BTG_ERR_LIMIT_CODE;
+      }
+      budget = int(std::min<unsigned long long>((unsigned long long)budget * 32, p.capacity));
     }
-    budget = int(std::min<unsigned long long>((unsigned long long)budget * 32, p.capacity));
-    // The retry list must not alias the list collectKilled writes next: copy it.
-    int rc2;
+    left -= nk;
     Params q = p;
     q.R = nk;
     q.budget = budget;
-    q.pass = p.pass + 1;
-    if ((rc2 = e.ensure(e.retry, size_t(nk) * 4, err))) return rc2;
-    BTG_TRY(hipMemcpyAsync(e.retry.ptr, e.list.ptr, size_t(nk) * 4, hipMemcpyDeviceToDevice, e.stream));
-    q.rootList = static_cast<const int*>(e.retry.ptr);
+    q.pass = ++p.pass;
+    q.rootList = static_cast<const int*>(e.list.ptr);
     info.retries++;
     if ((rc = runPass(e, q, info, err))) return rc;
     if ((rc = finalize(q))) return rc;
-    p.reserve = q.reserve;
-    p.pass = q.pass;
-    p.rootList = q.rootList;
-    p.R = q.R;
+    whole = true;
   }
   return 0;
 }

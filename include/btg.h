@@ -157,7 +157,7 @@ typedef struct {
   double totalSeconds;    /* host wall time of the call */
   int rounds;
   int maxQueue;
-  int killedRoots;        /* roots that went over budget in the first pass */
+  int killedRoots;        /* roots that the first pass abandoned: over budget, or without room in a queue */
   int retryPasses;        /* extra GPU passes that traced them exactly */
   btg_trace_stats stats;  /* beam counters (engine-independent) */
   btg_trace_stats rayStats;
