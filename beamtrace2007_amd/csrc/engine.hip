@@ -1166,7 +1166,8 @@ __device__ __forceinline__ int highestBit(uint64_t x) { return 63 - __builtin_cl
 // cycles per code region, summed into p.cycles[0..8). PHASE_MARK(k) charges
 // the time since the previous mark to region k: 0 refill, 1 descend, 2 climb
 // (parent walk), 3 climb (child box test), 4 output emit, 5 triangle tests,
-// 6 queue appends, 7 the rest of the traversal loop.
+// 6 queue appends, 7 the rest of the traversal loop. In a fused round 6 also holds
+// what a wave does between two traces: clips, integrals, the hand-over.
 enum { kPhRefill, kPhDescend, kPhWalk, kPhBox, kPhEmit, kPhTest, kPhAppend, kPhRest, kPhases };
 #ifdef BTG_PHASE_CYCLES
 struct PhaseClock {
@@ -2013,6 +2014,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
   if (n > 0) {
     Cnt cnt;
     cnt.zero();
+    PHASE_INIT();
     const Deal dl = dealOf();
     char* const ws = p.ws + size_t(dl.wave) * kWsBytes;
     Rec* const ts = reinterpret_cast<Rec*>(ws);
@@ -2078,12 +2080,15 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
             if (tsN > 0 || !exhausted) continue;
             break;
           }
+          PHASE_MARK(kPhRefill);
           if (exhausted) ++late;
           int res = kContinue;
-          if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt, wsh);
+          if (active) res = advance<App>(p, c, r, w, ss, path, bounds, cnt, wsh PHASE_PASS);
+          PHASE_MARK(kPhRest);
           const bool want = active && res == kContinue;
           const int cr = coopTest<App>(p, c, r, w, ss, want, cnt, mboxLds, bounds);
           if (want) res = cr;
+          PHASE_MARK(kPhTest);
           if (active) {
             if (res == kFinished) liveSub(p, r.root, 1);
             if (res != kContinue) active = false;
@@ -2109,6 +2114,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
             if (room) tsN += __popcll(busy);
             break;
           }
+          PHASE_MARK(kPhAppend);
         }
       }
       __threadfence_block();
@@ -2149,11 +2155,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))
         for (int k = lane(); k < tsN; k += kWave) toQueue(p, nxt, base + k, ts[k]);
         tsN = 0;
       }
+      PHASE_MARK(kPhAppend);
       if (tsN == 0 && exhausted) break;
       // a wave busy with its own stack learns here that the queue has run dry
       if (!exhausted && !first)
         exhausted = statics + *(volatile int*)&p.st->head[kHeadTrace] >= n;
     }
+    PHASE_FLUSH();
     flushCnt(p, cnt);
   }
   finishRound(p, cur);

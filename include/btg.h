@@ -168,7 +168,8 @@ typedef struct {
   int kernelLaunches[5];
   /* builds with -DBTG_PHASE_CYCLES: trace-loop clocks spent refilling,
    * descending, climbing (parent walk, child box test), emitting, testing
-   * triangles, appending and in the rest of the traversal (soft shadows) */
+   * triangles, appending (in rounds of one launch: and clipping and integrating)
+   * and in the rest of the traversal (soft shadows) */
   uint64_t phaseCycles[8];
 } btg_run_info;
 
