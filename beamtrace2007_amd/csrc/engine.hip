@@ -195,7 +195,7 @@ struct Params {
   unsigned long long capacity;
   Rec* tq[2];
   Rec* sq;
-  char* ws;  // fused passes: kWsBytes of buffers per wave of the grid (null: rounds of separate launches)
+  char* ws;  // fused rounds: kWsBytes of buffers per wave of the grid (null: none so far)
   RootQ* roots;
   int* live;
   int* state;
@@ -3281,8 +3281,9 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
             gS = residentGrid(e, splitKernel<App>), gH = residentGrid(e, shadeKernel);
   const bool shade = isSoft(App) && p.exact;
   const int gW = residentGrid(e, waveKernel<App>);
-  if (int rc = e.ensure(e.ws, size_t(gW) * (kBlock / kWave) * kWsBytes, err)) return rc;
-  p.ws = static_cast<char*>(e.ws.ptr);
+  // The waves' stacks (100 KB each, 205 MB for 2048 resident waves) come with the
+  // first fused round; without room for them all rounds run as separate launches.
+  bool stacks = true;
   // A first run admits more roots at once than their budgets would fit: what
   // matters is that the queue fills the device (with whole budgets reserved,
   // sixteen blob and atrium jobs ran 832 rounds at 1.6 waves per SIMD, 878 ms;
@@ -3330,9 +3331,14 @@ int runPassApp(Engine& e, Params& p, RunInfo& info, std::string& err) {
   int rounds = 0;
   for (;;) {
     const int par = rounds & 1;
-    const bool fused = queued < kDenseRecs;
+    if (stacks && !p.ws && queued < kDenseRecs) {
+      std::string none;
+      stacks = e.ensure(e.ws, size_t(gW) * (kBlock / kWave) * kWsBytes, none) == 0;
+      p.ws = static_cast<char*>(e.ws.ptr);
+    }
+    const bool fused = stacks && queued < kDenseRecs;
     // a queue not far above the line is looked at again soon: it may be shrinking
-    const int most = fused ? kFusedCheck : (queued < 8 * kDenseRecs ? 2 : e.opt.roundsPerCheck);
+    const int most = fused ? kFusedCheck : (stacks && queued < 8 * kDenseRecs ? 2 : e.opt.roundsPerCheck);
     const int k = std::max(1, std::min(e.opt.roundsPerCheck, most));
     if (graphs && k == e.opt.roundsPerCheck && !fused) {  // shorter groups are launched directly
       if (!gr.exec[par]) {

@@ -1,0 +1,98 @@
+"""Calls on a device that has room for their queues and outputs but not for the
+buffers that only make them faster: they go on without those, with the same
+results. Each case runs in a process of its own, in which the library's hipMalloc
+is one with a limit (tests/native/alloc_limit.c), once without and once with it."""
+import ctypes
+import os
+import shutil
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+class Limit:
+    """The process's hipMalloc (only in the processes that this module starts)."""
+
+    def __init__(self, path):
+        self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.lib.alloc_limit.argtypes = [ctypes.c_size_t]
+        self.lib.alloc_refuse.argtypes = [ctypes.c_int, ctypes.c_size_t]
+
+    def bytes(self, n):
+        self.lib.alloc_limit(n)
+
+    def refuse(self, sizes):
+        for i, n in enumerate(sizes):
+            self.lib.alloc_refuse(i, n)
+
+    def refusals(self):
+        return self.lib.alloc_refusals()
+
+
+def setup(name, W, H, **options):
+    from beamtrace2007_amd.gpu import GpuRenderer
+    from beamtrace2007_amd.host import camera
+    from conftest import load_scene
+    s, _, _, sp = load_scene(name)
+    r = GpuRenderer(s)
+    if options:
+        r.set_options(**options)
+    return r, camera(sp["view"], W, H), sp
+
+
+def same(a, b):
+    return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def wave_stacks(limit):
+    """The wave stacks (100 KB for each of 2048 waves) in passes of every kind."""
+    W, H = 70, 45
+    def run(limited):
+        if limited:
+            limit.bytes(100 << 20)  # the queues of this capacity and the output lists are smaller
+        r, cam, sp = setup("room", W, H, capacity=65536)
+        p, _ = r.primary(cam, W, H, tile=8)
+        q, _ = r.point_shadows(cam, W, H, p, sp["point_light"])
+        out = [p, q]
+        for precision in (0, 1):
+            r.set_options(precision=precision)
+            g = r.soft_shadows(cam, W, H, sp["area_light"], exact=True)
+            out += [g[f] for f in ("tri", "vis", "E", "Eu")]
+        r.close()
+        return out
+    return run
+
+
+CASES = {"wave_stacks": wave_stacks}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_calls_go_on_without(require_gpu, tmp_path, case):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    shim = str(tmp_path / "alloc_limit.so")
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", os.path.join(HERE, "native", "alloc_limit.c"), "-o", shim, "-ldl"],
+                   check=True, capture_output=True, timeout=60)
+    print(f"without room: {case}", flush=True)
+    out = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), shim, case], capture_output=True, text=True,
+                         timeout=100)
+    assert out.returncode == 0, out.stdout[-2000:] + out.stderr[-2000:]
+    assert out.stdout.splitlines()[-1] == "ok"
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, HERE)
+    import conftest  # noqa: F401  (the repository's root on the path)
+    lim = Limit(sys.argv[1])
+    run = CASES[sys.argv[2]](lim)
+    want = run(False)
+    assert lim.refusals() == 0
+    got = run(True)
+    print("allocations refused:", lim.refusals(), flush=True)
+    assert lim.refusals() > 0
+    assert same(want, got)
+    print("ok", flush=True)
