@@ -4390,15 +4390,15 @@ __global__ void compactPolys(const OutPoly* polys, const int* root, const int* t
 // equals their root's last pass. Canonical lists are sorted on the device:
 // primary and point shadows of the conference hall (220K and 230K polygons at
 // 640 x 481) take 21.8 ms, and 30.7 ms with the lists sorted on eight host
-// threads and their tags filtered there.
+// threads and their tags filtered there. Without room for the copies that
+// takes (44 B per polygon to filter, 52 B to sort), the host does it.
 int takePolys(Engine& e, bool filter, bool canonical, PolyList& polys, std::string& err) {
   int n = std::max(0, std::min(e.hostState->outCount, int(e.out.bytes / sizeof(OutPoly))));
   const OutPoly* src = static_cast<const OutPoly*>(e.out.ptr);
-  int rc;
   polys.clear();
   if (n == 0) return 0;
-  if (filter) {
-    if ((rc = e.ensure(e.valid, size_t(n) * sizeof(OutPoly), err)) || (rc = e.ensure(e.listCount, 4, err))) return rc;
+  std::string none;
+  if (filter && !e.ensure(e.valid, size_t(n) * sizeof(OutPoly), none)) {
     clearInt<<<1, 64, 0, e.stream>>>(static_cast<int*>(e.listCount.ptr));
     compactPolys<<<(n + 255) / 256, 256, 0, e.stream>>>(src, static_cast<const int*>(e.outRoot.ptr),
                                                         static_cast<const int*>(e.outTag.ptr),
@@ -4409,12 +4409,11 @@ int takePolys(Engine& e, bool filter, bool canonical, PolyList& polys, std::stri
     BTG_TRY(hipMemcpyAsync(&n, e.listCount.ptr, 4, hipMemcpyDeviceToHost, e.stream));
     BTG_TRY(hipStreamSynchronize(e.stream));
     src = static_cast<const OutPoly*>(e.valid.ptr);
+    filter = false;
     if (n == 0) return 0;
   }
-  if (canonical && n > 1) {
-    if ((rc = e.ensure(e.order, size_t(n) * 2 * sizeof(int), err)) ||
-        (rc = e.ensure(e.sorted, size_t(n) * sizeof(OutPoly), err)))
-      return rc;
+  if (canonical && !filter && n > 1 && !e.ensure(e.order, size_t(n) * 2 * sizeof(int), none) &&
+      !e.ensure(e.sorted, size_t(n) * sizeof(OutPoly), none)) {
     int* a = static_cast<int*>(e.order.ptr);
     int* b = a + n;
     sortBlocks<<<(n + kSortBlock - 1) / kSortBlock, kSortBlock, 0, e.stream>>>(src, n, a);
@@ -4424,10 +4423,27 @@ int takePolys(Engine& e, bool filter, bool canonical, PolyList& polys, std::stri
         src, a, n, static_cast<OutPoly*>(e.sorted.ptr));
     BTG_TRY(hipGetLastError());
     src = static_cast<const OutPoly*>(e.sorted.ptr);
+    canonical = false;
   }
   polys.resize(size_t(n));
   BTG_TRY(hipMemcpyAsync(polys.data(), src, sizeof(OutPoly) * size_t(n), hipMemcpyDeviceToHost, e.stream));
+  std::vector<int> root, tag, epoch;
+  if (filter) {
+    root.resize(size_t(n));
+    tag.resize(size_t(n));
+    epoch.resize(e.epoch.bytes / sizeof(int));
+    BTG_TRY(hipMemcpyAsync(root.data(), e.outRoot.ptr, root.size() * sizeof(int), hipMemcpyDeviceToHost, e.stream));
+    BTG_TRY(hipMemcpyAsync(tag.data(), e.outTag.ptr, tag.size() * sizeof(int), hipMemcpyDeviceToHost, e.stream));
+    BTG_TRY(hipMemcpyAsync(epoch.data(), e.epoch.ptr, epoch.size() * sizeof(int), hipMemcpyDeviceToHost, e.stream));
+  }
   BTG_TRY(hipStreamSynchronize(e.stream));
+  if (filter) {
+    size_t kept = 0;
+    for (size_t i = 0; i < size_t(n); ++i)
+      if (tag[i] == epoch[size_t(root[i])]) polys[kept++] = polys[i];
+    polys.resize(kept);
+  }
+  if (canonical) std::sort(polys.begin(), polys.end(), polyLess);
   return 0;
 }
 

@@ -67,7 +67,30 @@ def wave_stacks(limit):
     return run
 
 
-CASES = {"wave_stacks": wave_stacks}
+def lists(limit, **options):
+    """Canonical polygon lists where nothing can be allocated beyond what the passes hold: sorted, and with a small
+    budget (roots traced again) filtered, on the host."""
+    W = H = 48
+    def run(limited):
+        r, cam, sp = setup("plant", W, H)
+        p, _ = r.primary(cam, W, H, tile=16, canonical=False)
+        r.point_shadows(cam, W, H, p, sp["point_light"], canonical=False)
+        if options:
+            r.set_options(**options)
+        if limited:
+            limit.bytes(1)
+        p, info = r.primary(cam, W, H, tile=16)
+        q, info2 = r.point_shadows(cam, W, H, p, sp["point_light"])
+        assert len(p) > 256 and len(q) > 256  # more than a block of the device's sort
+        for i in (info, info2):
+            assert (i["retry_passes"] > 0) == bool(options)
+        r.close()
+        return [p, q]
+    return run
+
+
+CASES = {"wave_stacks": wave_stacks, "sorted_lists": lists,
+         "filtered_lists": lambda limit: lists(limit, primary_budget=4, budget=4)}
 
 
 @pytest.mark.gpu
