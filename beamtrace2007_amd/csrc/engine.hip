@@ -3785,17 +3785,24 @@ int softFp64(Engine& e, Params& p, size_t np, std::string& err) {
   using T2 = fp64::Tracer<384, 256>;
   constexpr size_t kBlock0 = size_t(T0::kWords) * 64 * 8, kBlock1 = size_t(T1::kWords) * 64 * 8,
                    kBlock2 = size_t(T2::kWords) * 64 * 8;
-  const size_t cus = size_t(std::max(e.cus, 1)), maxBlocks = cus * 4 * kFp64Waves;
-  const size_t blocks0 = std::min(np, maxBlocks);  // (its memory: less than blocks2 takes)
-  const size_t blocks1 = std::min((16 * np + 63) / 64, maxBlocks);
-  // every level fills the device's SIMDs (level 2 on one wave per CU took 1.35 times as long on the plant)
-  const size_t blocks2 = std::min((256 * np + 63) / 64, maxBlocks);
+  const size_t cus = size_t(std::max(e.cus, 1));
   const size_t cap2 = std::min<size_t>(16 * np, size_t(1) << 24);  // level-2 entries
   int rc;
-  if ((rc = e.ensure(e.fpMem, std::max({blocks0 * kBlock0, blocks1 * kBlock1, blocks2 * kBlock2}), err)) ||
-      (rc = e.ensure(e.fpList, 64 + (np + cap2) * sizeof(long long), err)) ||
+  if ((rc = e.ensure(e.fpList, 64 + (np + cap2) * sizeof(long long), err)) ||
       (rc = e.ensure(e.fpSum, 2 * np * sizeof(unsigned long long), err)))
     return rc;
+  // Every level fills the device's SIMDs (level 2 on one wave per CU took 1.35
+  // times as long on the plant), which takes 3.9 GB for level 2's pools; without
+  // room for that, half as many waves, down to one per CU.
+  size_t blocks0, blocks1, blocks2;
+  for (size_t most = cus * 4 * kFp64Waves;; most /= 2) {
+    blocks0 = std::min(np, most);
+    blocks1 = std::min((16 * np + 63) / 64, most);
+    blocks2 = std::min((256 * np + 63) / 64, most);
+    rc = e.ensure(e.fpMem, std::max({blocks0 * kBlock0, blocks1 * kBlock1, blocks2 * kBlock2}), err);
+    if (!rc) break;
+    if (rc != BTG_ERR_MEMORY_CODE || most / 2 < cus) return rc;
+  }
   uint64_t* mem = static_cast<uint64_t*>(e.fpMem.ptr);
   int* ctr = static_cast<int*>(e.fpList.ptr);  // next[3], outCount[2], failed
   long long* list1 = reinterpret_cast<long long*>(static_cast<char*>(e.fpList.ptr) + 64);

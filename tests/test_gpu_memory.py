@@ -89,8 +89,22 @@ def lists(limit, **options):
     return run
 
 
+def fp64_pools(limit, gib):
+    """FP64 soft shadows with room for the pools of half or a quarter of the waves that fill the device."""
+    W, H = 40, 30
+    def run(limited):
+        if limited:
+            limit.bytes(int(gib * (1 << 30)))
+        r, cam, sp = setup("room", W, H, precision=2)
+        g = r.soft_shadows(cam, W, H, sp["area_light"], exact=True)
+        r.close()
+        return [g[f] for f in ("tri", "vis", "E", "Eu")]
+    return run
+
+
 CASES = {"wave_stacks": wave_stacks, "sorted_lists": lists,
-         "filtered_lists": lambda limit: lists(limit, primary_budget=4, budget=4)}
+         "filtered_lists": lambda limit: lists(limit, primary_budget=4, budget=4),
+         "fp64_half": lambda limit: fp64_pools(limit, 2.0), "fp64_quarter": lambda limit: fp64_pools(limit, 1.0)}
 
 
 @pytest.mark.gpu
