@@ -2850,7 +2850,7 @@ __global__ void zeroWords(unsigned long long* w, size_t n) {
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) w[i] = 0;
 }
 
-// One level of FP64 soft shadows. Tasks: level 0, the pixels 0..numPix-1;
+// One level of FP64 soft shadows. Tasks: level 0, the numPix pixels from pix0 on;
 // level 1, 16 per entry of `in` (a pixel: the cells of its 4 x 4 grid);
 // level 2, 16 per entry (pixel << 4 | a level-1 cell: the 16 x 16 grid's
 // cells inside it). Each lane takes tasks from `next` until none is left,
@@ -2867,7 +2867,7 @@ __global__ void zeroWords(unsigned long long* w, size_t n) {
 // lanes the same.
 template <int Pn, int Kn, int Level>
 __global__ void __launch_bounds__(64, kFp64Waves)
-    fp64CellKernel(Params p, int numPix, const long long* in, const int* inCount, int inCap, int* next, uint64_t* mem,
+    fp64CellKernel(Params p, int pix0, int numPix, const long long* in, const int* inCount, int inCap, int* next, uint64_t* mem,
                    long long* out, int* outCount, int outCap, unsigned long long* visSum, unsigned long long* gSum,
                    int* failed) {
   using TR = fp64::Tracer<Pn, Kn>;
@@ -2879,7 +2879,7 @@ __global__ void __launch_bounds__(64, kFp64Waves)
   for (; int(threadIdx.x) < lanes;) {
     const int t = atomicAdd(next, 1);
     if (t >= tasks) break;
-    int pix = t, cx = 0, cy = 0;
+    int pix = pix0 + t, cx = 0, cy = 0;
     if (Level > 0) {
       const long long e = in[t >> 4];
       const int s = t & 15;
@@ -3772,13 +3772,21 @@ Options& engineOptions(Engine* e) { return e->opt; }
 
 namespace {
 
+// Pixels whose cells are traced together (levels 0 to 2), at most: their list of
+// overflowed level-1 cells (8 B each) holds all 16 of every pixel, so no image is
+// too large for it. (With one list of 2^24 for a whole call, the plant's 2.6
+// entries a pixel at a work cap of 512 fill it at 6.5M pixels; at 2048 it was
+// 0.8.) The levels' tails come once per chunk: the atrium at 1400 x 1400 took 635 ms
+// in one chunk and 687 ms in two. 2^22 keeps the task numbers within 31 bits.
+constexpr size_t kFp64Chunk = size_t(1) << 22, kFp64ChunkLeast = size_t(1) << 20;
+
 // FP64 soft shadows of every pixel of a batch (after its primary pass), in
 // three levels of cells (fp64CellKernel): the whole root with pools of 64
 // beams and the work cap; the 4 x 4 cells of the roots that overflowed, with
 // 128 beams and the cap; the 16 x 16 cells inside those that overflowed
 // again, with 384 beams and no cap. The levels run back to back on the stream
-// (each reads its task count from the device); one synchronisation at the end
-// reads the cells that overflowed their last level.
+// (each reads its task count from the device), chunk after chunk; one
+// synchronisation at the end reads the cells that overflowed their last level.
 int softFp64(Engine& e, Params& p, size_t np, std::string& err) {
   using T0 = fp64::Tracer<64, 64>;
   using T1 = fp64::Tracer<kFp64Pool1, kFp64Pool1>;
@@ -3786,48 +3794,56 @@ int softFp64(Engine& e, Params& p, size_t np, std::string& err) {
   constexpr size_t kBlock0 = size_t(T0::kWords) * 64 * 8, kBlock1 = size_t(T1::kWords) * 64 * 8,
                    kBlock2 = size_t(T2::kWords) * 64 * 8;
   const size_t cus = size_t(std::max(e.cus, 1));
-  const size_t cap2 = std::min<size_t>(16 * np, size_t(1) << 24);  // level-2 entries
   int rc;
-  if ((rc = e.ensure(e.fpList, 64 + (np + cap2) * sizeof(long long), err)) ||
-      (rc = e.ensure(e.fpSum, 2 * np * sizeof(unsigned long long), err)))
-    return rc;
+  size_t chunk = std::min(np, kFp64Chunk), cap2;  // pixels, level-2 entries
+  for (;; chunk = (chunk + 1) / 2) {  // smaller chunks without room for their lists
+    cap2 = 16 * chunk;
+    rc = e.ensure(e.fpList, 64 + (chunk + cap2) * sizeof(long long), err);
+    if (!rc) break;
+    if (rc != BTG_ERR_MEMORY_CODE || chunk <= kFp64ChunkLeast) return rc;
+  }
+  if ((rc = e.ensure(e.fpSum, 2 * np * sizeof(unsigned long long), err))) return rc;
   // Every level fills the device's SIMDs (level 2 on one wave per CU took 1.35
   // times as long on the plant), which takes 3.9 GB for level 2's pools; without
   // room for that, half as many waves, down to one per CU.
   size_t blocks0, blocks1, blocks2;
   for (size_t most = cus * 4 * kFp64Waves;; most /= 2) {
-    blocks0 = std::min(np, most);
-    blocks1 = std::min((16 * np + 63) / 64, most);
-    blocks2 = std::min((256 * np + 63) / 64, most);
+    blocks0 = std::min(chunk, most);
+    blocks1 = std::min((16 * chunk + 63) / 64, most);
+    blocks2 = std::min((256 * chunk + 63) / 64, most);
     rc = e.ensure(e.fpMem, std::max({blocks0 * kBlock0, blocks1 * kBlock1, blocks2 * kBlock2}), err);
     if (!rc) break;
     if (rc != BTG_ERR_MEMORY_CODE || most / 2 < cus) return rc;
   }
   uint64_t* mem = static_cast<uint64_t*>(e.fpMem.ptr);
-  int* ctr = static_cast<int*>(e.fpList.ptr);  // next[3], outCount[2], failed
+  int* ctr = static_cast<int*>(e.fpList.ptr);  // next[3], outCount[2] of a chunk; from 8 on: failed
+  int* failedCells = ctr + 8;
   long long* list1 = reinterpret_cast<long long*>(static_cast<char*>(e.fpList.ptr) + 64);
-  long long* list2 = list1 + np;
+  long long* list2 = list1 + chunk;
   unsigned long long* visSum = static_cast<unsigned long long*>(e.fpSum.ptr);
   unsigned long long* gSum = visSum + np;
-  zeroWords<<<1, 64, 0, e.stream>>>(reinterpret_cast<unsigned long long*>(ctr), 8);
+  zeroWords<<<1, 64, 0, e.stream>>>(reinterpret_cast<unsigned long long*>(failedCells), 1);
   zeroWords<<<unsigned(std::min<size_t>((2 * np + 255) / 256, 4096)), 256, 0, e.stream>>>(visSum, 2 * np);
-  const int n = int(np);
-  int lt = e.beginLaunch(1);
-  fp64CellKernel<64, 64, 0><<<unsigned(blocks0), 64, 0, e.stream>>>(p, n, nullptr, nullptr, 0, ctr, mem, list1,
-                                                                    ctr + 3, n, visSum, gSum, ctr + 5);
-  e.endLaunch(lt);
-  lt = e.beginLaunch(1);
-  fp64CellKernel<kFp64Pool1, kFp64Pool1, 1><<<unsigned(blocks1), 64, 0, e.stream>>>(p, n, list1, ctr + 3, n, ctr + 1, mem, list2,
-                                                                      ctr + 4, int(cap2), visSum, gSum, ctr + 5);
-  e.endLaunch(lt);
-  lt = e.beginLaunch(1);
-  fp64CellKernel<384, 256, 2><<<unsigned(blocks2), 64, 0, e.stream>>>(p, n, list2, ctr + 4, int(cap2), ctr + 2, mem,
-                                                                      nullptr, nullptr, 0, visSum, gSum, ctr + 5);
-  e.endLaunch(lt);
-  fp64FinishKernel<<<unsigned((np + 255) / 256), 256, 0, e.stream>>>(p, n, visSum, gSum);
+  for (size_t at = 0; at < np; at += chunk) {
+    const int pix0 = int(at), n = int(std::min(chunk, np - at));
+    zeroWords<<<1, 64, 0, e.stream>>>(reinterpret_cast<unsigned long long*>(ctr), 4);
+    int lt = e.beginLaunch(1);
+    fp64CellKernel<64, 64, 0><<<unsigned(blocks0), 64, 0, e.stream>>>(p, pix0, n, nullptr, nullptr, 0, ctr, mem, list1,
+                                                                      ctr + 3, n, visSum, gSum, failedCells);
+    e.endLaunch(lt);
+    lt = e.beginLaunch(1);
+    fp64CellKernel<kFp64Pool1, kFp64Pool1, 1><<<unsigned(blocks1), 64, 0, e.stream>>>(
+        p, pix0, n, list1, ctr + 3, n, ctr + 1, mem, list2, ctr + 4, int(cap2), visSum, gSum, failedCells);
+    e.endLaunch(lt);
+    lt = e.beginLaunch(1);
+    fp64CellKernel<384, 256, 2><<<unsigned(blocks2), 64, 0, e.stream>>>(
+        p, pix0, n, list2, ctr + 4, int(cap2), ctr + 2, mem, nullptr, nullptr, 0, visSum, gSum, failedCells);
+    e.endLaunch(lt);
+  }
+  fp64FinishKernel<<<unsigned((np + 255) / 256), 256, 0, e.stream>>>(p, int(np), visSum, gSum);
   BTG_TRY(hipGetLastError());
   int failed = 0;
-  BTG_TRY(hipMemcpyAsync(&failed, ctr + 5, 4, hipMemcpyDeviceToHost, e.stream));
+  BTG_TRY(hipMemcpyAsync(&failed, failedCells, 4, hipMemcpyDeviceToHost, e.stream));
   BTG_TRY(hipStreamSynchronize(e.stream));
   if (failed > 0) {
     err = std::to_string(failed) + " cell(s) of 1/256 of a pixel's light need more than 384 live beams in FP64 mode";

@@ -102,9 +102,23 @@ def fp64_pools(limit, gib):
     return run
 
 
+def fp64_lists(limit):
+    """An FP64 image of more than 2^22 pixels without room for the cell lists of 2^22 (17 entries of 8 B a pixel)."""
+    W = H = 2049
+    def run(limited):
+        if limited:
+            limit.refuse([64 + (17 << 22) * 8])
+        r, cam, sp = setup("room", W, H, precision=2)
+        g = r.soft_shadows(cam, W, H, sp["area_light"], exact=True)
+        r.close()
+        return [g[f] for f in ("tri", "vis", "E", "Eu")]
+    return run
+
+
 CASES = {"wave_stacks": wave_stacks, "sorted_lists": lists,
          "filtered_lists": lambda limit: lists(limit, primary_budget=4, budget=4),
-         "fp64_half": lambda limit: fp64_pools(limit, 2.0), "fp64_quarter": lambda limit: fp64_pools(limit, 1.0)}
+         "fp64_lists": fp64_lists, "fp64_half": lambda limit: fp64_pools(limit, 2.0),
+         "fp64_quarter": lambda limit: fp64_pools(limit, 1.0)}
 
 
 @pytest.mark.gpu
