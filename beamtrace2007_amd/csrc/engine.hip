@@ -3057,7 +3057,7 @@ struct SceneRec {
   int numTris = 0;
   uint32_t numVerts = 0;
   float offset = 0, offsetGuard = 0;
-  uint64_t ancEntries = 0;  // ancestor list entries of its leaves
+  uint64_t ancEntries = 0;  // ancestor list entries of its leaves (0: no lists)
   uint32_t nodeBase = 0, refBase = 0, triBase = 0, vertBase = 0;  // placement in the arena
 };
 
@@ -3643,6 +3643,8 @@ int rebuildArena(Engine& e, std::string& err) {
       (void)hipGetLastError();
     }
   }
+  if (!sv.anc)
+    for (SceneRec& sr : e.scenes) sr.ancEntries = 0;
   const SceneRec& s0 = e.scenes[0];
   sv.bounds = s0.bounds;
   sv.numTris = s0.numTris;

@@ -67,6 +67,38 @@ def wave_stacks(limit):
     return run
 
 
+def ancestor_lists(limit, name, **options):
+    """Climbs by parent links: a scene without its leaves' ancestor lists (8 B per leaf and level), which its bytes
+    then don't count. Images, lists and counters."""
+    from conftest import load_scene
+    nodes = load_scene(name)[2]["nodes"]
+    depth = np.zeros(len(nodes), np.int64)
+    for i in np.flatnonzero(nodes["data"] & 3 != 3):  # children follow their parent
+        depth[i + 1] = depth[nodes["data"][i] >> 2] = depth[i] + 1
+    size = 8 * int(depth[nodes["data"] & 3 == 3].sum())
+    W, H = 75, 50
+    def run(limited):
+        if limited:
+            limit.refuse([size])
+        r, cam, sp = setup(name, W, H, **options)
+        p, i = r.primary(cam, W, H, tile=16)
+        q, j = r.point_shadows(cam, W, H, p, sp["point_light"])
+        out, infos = [p, q], [i, j]
+        for precision in (0, 1):
+            r.set_options(precision=precision)
+            g = r.soft_shadows(cam, W, H, sp["area_light"], exact=True)
+            out += [g[f] for f in ("tri", "vis", "E", "Eu")]
+            infos.append(g["info"])
+        assert all(i["killed_roots"] == 0 for i in infos)
+        # a float sum over waves, in whatever order they end, is the one counter that may differ
+        counters = [{k: v for k, v in i["stats"].items() if k != "droppedArea"} for i in infos]
+        out.append(np.array([list(c.values()) for c in counters]))
+        out.append(r.scene_bytes(0) + (size if limited else 0))
+        r.close()
+        return out
+    return run
+
+
 def lists(limit, **options):
     """Canonical polygon lists where nothing can be allocated beyond what the passes hold: sorted, and with a small
     budget (roots traced again) filtered, on the host."""
@@ -115,7 +147,10 @@ def fp64_lists(limit):
     return run
 
 
-CASES = {"wave_stacks": wave_stacks, "sorted_lists": lists,
+CASES = {"wave_stacks": wave_stacks,
+         "ancestors_atrium": lambda limit: ancestor_lists(limit, "atrium"),
+         "ancestors_plant": lambda limit: ancestor_lists(limit, "plant", leaf_cap=1),
+         "sorted_lists": lists,
          "filtered_lists": lambda limit: lists(limit, primary_budget=4, budget=4),
          "fp64_lists": fp64_lists, "fp64_half": lambda limit: fp64_pools(limit, 2.0),
          "fp64_quarter": lambda limit: fp64_pools(limit, 1.0)}
