@@ -4696,23 +4696,56 @@ __device__ __forceinline__ void rasterPixel(const RasterArgs& a, size_t at, int 
     atomicMax(&a.ids[at], tri);  // polygons sort by tri first: the canonical last writer
 }
 
-// A workgroup takes 256 polygons and deals their rows to its threads, so that
-// one launch needs no scan over the whole list and no count on the host before
-// the next one. Polygons of more than kTallRows rows would leave a workgroup's
-// threads behind the others': they go to a list that rasterTallKernel takes a
-// row per wave, 64 pixels at a time. Bound by latency at ordinary sizes (a few
+// The spans of a wave's 64 lanes (x0 > x1: none; all lanes call it): narrow ones
+// each by its own lane, wide ones one after the other by the whole wave, those
+// between eight at a time by eight lanes each. A lane's own pixels go to 64
+// lines at once, 64 lanes' of one span to two or four, but spans in turn are a chain: of
+// 16 pixels in turn by the whole wave the conference hall's ids took 81 us a call
+// instead of 53. 64000 polygons of 30 rows into 1024 x 1024 ids, spans of 1, 5,
+// 10, 60 and 400 pixels: 0.10 / 0.39 / 0.75 / 4.4 / 26.8 ms each by its lane, 0.10 /
+// 0.15 / 0.21 / 0.39 / 2.0 ms now. A mask's plain stores are worth it from 16
+// pixels on (from 4: the hall's mask 54 us instead of 48).
+constexpr int kNarrowIds = 4, kNarrowMask = 16, kWideSpan = 32, kSpanLanes = 8;
+__device__ __forceinline__ void rasterSpans(const RasterArgs& a, int y, int x0, int x1, int tri) {
+  const int width = x1 - x0 + 1, narrow = a.shadow ? kNarrowMask : kNarrowIds;
+  if (width <= narrow)
+    for (int x = x0; x <= x1; ++x) rasterPixel(a, size_t(y) * size_t(a.W) + size_t(x), tri);
+  for (uint64_t m = __ballot(width >= kWideSpan); m; m &= m - 1) {
+    const int l = __builtin_ctzll(m);
+    const size_t row = size_t(__shfl(y, l, kWave)) * size_t(a.W);
+    const int end = __shfl(x1, l, kWave), t = __shfl(tri, l, kWave);
+    for (int x = __shfl(x0, l, kWave) + lane(); x <= end; x += kWave) rasterPixel(a, row + size_t(x), t);
+  }
+  const bool between = width > narrow && width < kWideSpan;
+  const uint64_t m = __ballot(between);
+  if (!m) return;
+  const int mine = between ? x1 : x0 - 1;
+  for (int g = 0; g < kWave; g += kWave / kSpanLanes) {
+    if (!((m >> g) & ((1u << (kWave / kSpanLanes)) - 1))) continue;
+    const int l = g + lane() / kSpanLanes;
+    const size_t row = size_t(__shfl(y, l, kWave)) * size_t(a.W);
+    const int end = __shfl(mine, l, kWave), t = __shfl(tri, l, kWave);
+    for (int x = __shfl(x0, l, kWave) + lane() % kSpanLanes; x <= end; x += kSpanLanes) rasterPixel(a, row + size_t(x), t);
+  }
+}
+
+// A workgroup takes `per` polygons (rasterPer) and deals their rows to its
+// threads, so that one launch needs no scan over the whole list and no count on
+// the host before the next one. Polygons of more than kTallRows rows would leave
+// a workgroup behind the others: they go to a list that rasterTallKernel takes
+// in slices of rows. Bound by latency at ordinary sizes (a few
 // rows and pixels per polygon). 230K polygons of the conference hall into 512 x
 // 512 ids: 58 us for the call, 69 us in five launches with a scan over the list
 // and a read-back of its total before the last.
 constexpr int kRasterBlock = 256, kTallRows = 32, kTallSlices = 16;
-__global__ void __launch_bounds__(kRasterBlock) rasterKernel(RasterArgs a) {
+__global__ void __launch_bounds__(kRasterBlock) rasterKernel(RasterArgs a, int per) {
   __shared__ int offs[kRasterBlock];
   __shared__ int waveSums[kRasterBlock / 64];
-  const int base = int(blockIdx.x) * kRasterBlock, i = base + int(threadIdx.x);
+  const int base = int(blockIdx.x) * per, i = base + int(threadIdx.x);
   int rows = 0;
   OutPoly pg;
   RasterEdges r;
-  if (i < a.n) rows = rasterRows(a, i, pg, r);
+  if (int(threadIdx.x) < per && i < a.n) rows = rasterRows(a, i, pg, r);
   if (rows > kTallRows) {
     const uint64_t m = __ballot(1);
     const int leader = __builtin_ctzll(m);
@@ -4724,36 +4757,57 @@ __global__ void __launch_bounds__(kRasterBlock) rasterKernel(RasterArgs a) {
   int total;
   offs[threadIdx.x] = blockExclusiveScan(rows, waveSums, &total);
   __syncthreads();
-  for (int j = int(threadIdx.x); j < total; j += kRasterBlock) {
-    int lo = 0, hi = kRasterBlock - 1;  // the last polygon whose first row is <= j
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (offs[mid] <= j)
-        lo = mid;
-      else
-        hi = mid - 1;
+  for (int j0 = int(threadIdx.x) - lane(); j0 < total; j0 += kRasterBlock) {
+    const int j = j0 + lane();
+    int y = 0, x0 = 0, x1 = -1;
+    pg.tri = 0;
+    if (j < total) {
+      int lo = 0, hi = per - 1;  // the last polygon whose first row is <= j
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (offs[mid] <= j)
+          lo = mid;
+        else
+          hi = mid - 1;
+      }
+      if (rasterRows(a, base + lo, pg, r) > 0) {  // always: its rows were counted
+        y = r.y0 + (j - offs[lo]);
+        rasterSpan(r, y, a.W, x0, x1);
+      }
     }
-    if (rasterRows(a, base + lo, pg, r) == 0) continue;  // never: its rows were counted
-    const int y = r.y0 + (j - offs[lo]);
-    int x0, x1;
-    rasterSpan(r, y, a.W, x0, x1);
-    for (int x = x0; x <= x1; ++x) rasterPixel(a, size_t(y) * size_t(a.W) + size_t(x), pg.tri);
+    rasterSpans(a, y, x0, x1, pg.tri);
   }
 }
 
+// A wave takes a polygon's slice of rows, its lanes a row each. Few polygons are
+// cut into up to kTallSlices slices, dealt 4 or 16 rows at a time, so that they
+// spread over the device; many are taken whole, 64 rows at a time.
 __global__ void __launch_bounds__(kRasterBlock) rasterTallKernel(RasterArgs a) {
-  const int64_t waves = int64_t(gridDim.x) * (kRasterBlock / 64);
-  const int64_t units = int64_t(*a.count) * kTallSlices;
-  for (int64_t u = int64_t(blockIdx.x) * (kRasterBlock / 64) + threadIdx.x / 64; u < units; u += waves) {
+  const int64_t waves = int64_t(gridDim.x) * (kRasterBlock / 64), count = int64_t(*a.count);
+  const int slices = count * kTallSlices <= 2 * waves ? kTallSlices : int(max(int64_t(1), 2 * waves / max(count, int64_t(1))));
+  const int step = slices == kTallSlices ? 4 : (slices > 1 ? 16 : kWave);
+  for (int64_t u = int64_t(blockIdx.x) * (kRasterBlock / 64) + threadIdx.x / 64; u < count * slices; u += waves) {
     OutPoly pg;
     RasterEdges r;
-    if (rasterRows(a, a.tall[u / kTallSlices], pg, r) == 0) continue;
-    for (int y = r.y0 + int(u % kTallSlices); y <= r.y1; y += kTallSlices) {
-      int x0, x1;
-      rasterSpan(r, y, a.W, x0, x1);
-      for (int x = x0 + lane(); x <= x1; x += kWave) rasterPixel(a, size_t(y) * size_t(a.W) + size_t(x), pg.tri);
+    if (rasterRows(a, a.tall[u / slices], pg, r) == 0) continue;
+    for (int y0 = r.y0 + int(u % slices) * step; y0 <= r.y1; y0 += slices * step) {
+      const int y = y0 + lane();
+      int x0 = 0, x1 = -1;
+      if (lane() < step && y <= r.y1) rasterSpan(r, y, a.W, x0, x1);
+      rasterSpans(a, y, x0, x1, pg.tri);
     }
   }
+}
+
+// Polygons per workgroup: 256 of a long list; fewer of a shorter one, down to 8,
+// so that about four workgroups per CU share it and a thread has a row or two
+// also where each polygon has tens of rows. With 256 of every list a thousand
+// polygons ran on four workgroups: at 30 rows of 60 pixels 773 us, 36 us now (128 us
+// with a thread for every row of the whole list).
+int rasterPer(const Engine& e, int n) {
+  int per = 8;
+  while (per < kRasterBlock && (long long)per * std::max(e.cus, 1) * 4 < n) per *= 2;
+  return per;
 }
 
 // The rows of all polygons together, in *a.count.
@@ -4816,9 +4870,8 @@ int rasterInto(Engine& e, const HostCam& cam, const OutPoly* polys, const int* r
   fill();
   BTG_TRY(hipGetLastError());
   if (n <= 0) return 0;
-  const int blocks = (n + kRasterBlock - 1) / kRasterBlock;
   if (uint64_t(n) * uint64_t(cam.H) > 0xffffffffull) {  // only such a list can hold more rows than are taken
-    rasterCountKernel<<<std::min(blocks, 4096), kRasterBlock, 0, e.stream>>>(a);
+    rasterCountKernel<<<std::min((n + kRasterBlock - 1) / kRasterBlock, 4096), kRasterBlock, 0, e.stream>>>(a);
     BTG_TRY(hipGetLastError());
     unsigned long long total = 0;
     BTG_TRY(hipMemcpyAsync(&total, a.count, 8, hipMemcpyDeviceToHost, e.stream));
@@ -4829,7 +4882,8 @@ int rasterInto(Engine& e, const HostCam& cam, const OutPoly* polys, const int* r
     }
     fill();  // the count again
   }
-  rasterKernel<<<blocks, kRasterBlock, 0, e.stream>>>(a);
+  const int per = rasterPer(e, n);
+  rasterKernel<<<(n + per - 1) / per, kRasterBlock, 0, e.stream>>>(a, per);
   rasterTallKernel<<<std::max(e.cus, 1) * 4, kRasterBlock, 0, e.stream>>>(a);
   BTG_TRY(hipGetLastError());
   return 0;
