@@ -4639,6 +4639,13 @@ __device__ __forceinline__ void rasterSpan(const RasterEdges& r, int y, int W, i
   x1 = toIntHost(floor(xr - 0.5));
   x0 = x0 > 0 ? x0 : 0;
   x1 = x1 < W - 1 ? x1 : W - 1;
+  // None as (0, -1): x0 may be near INT_MAX here and x1 INT_MIN (an edge on either
+  // side of 2^31 pixels), where a width or x0 + lane() would wrap to a pixel far
+  // outside the image.
+  if (x0 > x1) {
+    x0 = 0;
+    x1 = -1;
+  }
 }
 
 // Exclusive scan of one value per thread across the block (wave64 shuffles,
