@@ -13,28 +13,32 @@ namespace btg {
 // place none. Caller's polygons reach the lists as they are (receivers that face
 // away from the light), NaN corners included.
 BTG_HD int orderOf(float a, float b) {
+  if (a == b) return 0;
   if (a < b) return -1;
   if (b < a) return 1;
   return int(a != a) - int(b != b);
 }
 
-// polyLess of the reference's canonical list: triangle, corner count, corners, area.
-BTG_HD bool polyLess(const OutPoly& a, const OutPoly& b) {
-  if (a.tri != b.tri) return a.tri < b.tri;
-  if (a.n != b.n) return a.n < b.n;
+// The reference's canonical order (polyLess): triangle, corner count, corners,
+// area; -1, 0 or 1 as orderOf.
+BTG_HD int polyOrder(const OutPoly& a, const OutPoly& b) {
+  if (a.tri != b.tri) return a.tri < b.tri ? -1 : 1;
+  if (a.n != b.n) return a.n < b.n ? -1 : 1;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     if (k >= a.n) break;
-    if (const int o = orderOf(a.x[k], b.x[k])) return o < 0;
-    if (const int o = orderOf(a.y[k], b.y[k])) return o < 0;
+    if (const int o = orderOf(a.x[k], b.x[k])) return o;
+    if (const int o = orderOf(a.y[k], b.y[k])) return o;
   }
-  return orderOf(a.area, b.area) < 0;
+  return orderOf(a.area, b.area);
 }
+BTG_HD bool polyLess(const OutPoly& a, const OutPoly& b) { return polyOrder(a, b) < 0; }
 
 // Whether polygon a, at place ia, goes before polygon b, at place ib: equal
 // polygons keep their order, so that no two share a place.
 BTG_HD bool goesBefore(const OutPoly& a, int ia, const OutPoly& b, int ib) {
-  return polyLess(a, b) || (ia < ib && !polyLess(b, a));
+  const int o = polyOrder(a, b);
+  return o < 0 || (o == 0 && ia < ib);
 }
 
 // How many of the sibling run's `count` polygons, at(0) to at(count - 1) in
@@ -46,7 +50,7 @@ BTG_HD int mergeBefore(const OutPoly& own, bool second, int count, At at) {
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     const OutPoly other = at(mid);
-    if (second ? !polyLess(own, other) : polyLess(other, own))
+    if (polyOrder(other, own) < int(second))
       lo = mid + 1;
     else
       hi = mid;
