@@ -427,10 +427,11 @@ int btg_autotune(btg_ctx* ctx, const btg_soft_job* jobs, int numJobs, int exact,
   // best value of a knob is kept before the next knob is tuned. No leaf cap
   // (0) is not tried: uncapped stragglers made every measured batch slower
   // (3x on the 64-job batch). The per-root budget is not tuned: it decides
-  // which roots are abandoned and traced again, and how many roots the queue
-  // capacity admits at once, so a scaled-down sample (fewer roots, retries
-  // weighing more) misjudges it: 2048 won on the quarter-side sample of the
-  // 64-job batch and lost by 7% on the batch itself.
+  // which roots are abandoned and traced again (not, since a first run
+  // reserves at most 128 records a root, how many run at once), so a scaled-down
+  // sample, in which retries weigh more, misjudges it: 2048 won on the
+  // quarter-side sample of the 64-job batch and lost by 7% on the batch itself
+  // (measured with whole budgets reserved).
   struct Knob {
     int btg::Options::*field;
     std::vector<int> values;

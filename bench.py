@@ -69,17 +69,16 @@ WORKLOADS = {
                          "coin, square side uniform 128..1024, light scale log-uniform 0.25..4"),
 }
 METRIC = "exact soft-shadow pixels/s, batched vs plain (1 GPU); p50/p99 request latency"
-# Measured HBM bytes per trace-kernel launch (rocprofv3 FETCH_SIZE + WRITE_SIZE,
-# scaled by a 256 MiB copy: the *_hbm_traffic.txt summaries under profiles/) and
-# the trace kernel's issue figures (rocprofv3 SQ counters: *_valu_busy.txt,
-# *_sq_counters.txt), valid only for the library build and schedule they were
-# measured with: keyed by the SHA-256 prefix of lib/libbtg.so and the schedule,
-# so that any kernel change or another schedule reports null, never a stale figure.
-TRAFFIC = {("0536bc727452f3d8", "plant", 512): 479315442}
-TRAFFIC_BATCH = {("0536bc727452f3d8", 1 << 28, 1024, 8, 8, False): 5057140028,
-                 ("0536bc727452f3d8", 1 << 28, 1024, 8, 4, False): 3980057483}
-ISSUE_BATCH = {("0536bc727452f3d8", 1 << 28, 1024, 8, 8, False): {"valu_busy": 0.843, "lane_utilisation": 0.259},
-               ("0536bc727452f3d8", 1 << 28, 1024, 8, 4, False): {"valu_busy": 0.845, "lane_utilisation": 0.263}}
+# Measured HBM bytes per trace launch (traceKernel and waveKernel, rocprofv3
+# FETCH_SIZE + WRITE_SIZE scaled by a 256 MiB copy) and the trace kernel's issue
+# figures (rocprofv3 SQ counters), both from the summaries under profiles/
+# (trace_batch64.txt, trace_plant512.txt), valid only for the library build and
+# schedule they were measured with: keyed by the SHA-256 prefix of lib/libbtg.so
+# and the schedule, so that any kernel change or another schedule reports null,
+# never a stale figure.
+TRAFFIC = {("110579ca862b6d84", "plant", 512): 784436338}
+TRAFFIC_BATCH = {("110579ca862b6d84", 1 << 28, 1024, 8, 8, False): 16296867049}
+ISSUE_BATCH = {("110579ca862b6d84", 1 << 28, 1024, 8, 8, False): {"valu_busy": 0.969, "lane_utilisation": 0.313}}
 
 
 def library_hash() -> str:

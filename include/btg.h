@@ -329,7 +329,11 @@ typedef struct btg_server btg_server;
 typedef struct {
   int64_t hbmBytes;    /* device memory for work in flight, split between two passes (0: 128 GiB, or 45% of the
                           device where that is less); a quarter of it holds the passes' queues, which set how
-                          many roots run at once */
+                          many roots run at once. Not counted in it: the engine of point requests and the one of
+                          requests traced again alone (or of FP64 batches), whose buffers come with their first
+                          request and stay: queues of at most the passes' capacity, output lists, 0.2 GB of wave
+                          stacks each; FP64 batches 3.9 GB of pools and up to 0.6 GB of cell lists (less where
+                          they do not fit) */
   int roundsPerStep;   /* wavefront rounds between host checks (0: 8) */
   int jobsPerPass;     /* request slots of one pass (0: 512) */
 } btg_server_config;
